@@ -290,7 +290,8 @@ __device__ __forceinline__ void lane_segment(const Params& p, int64_t s, int64_t
 // A wave-class segment in the row mapping reduced by a group of lanes that
 // together hold one row (lane `feature_lane` owns features feature_lane*VEC
 // .. +VEC): every lane walks all rows of the segment on its own, so no lane
-// waits for another; eight rows' loads in flight per lane.
+// waits for another; eight rows' loads in flight per lane (four with a
+// mask of four or more words a lane: eight spilled 22 words per lane).
 template <int OP, class T, int VEC, bool MASK>
 __device__ __forceinline__ void group_segment(const Params& p, int64_t s, int64_t start, int64_t end,
                                               int feature_lane) {
@@ -298,14 +299,15 @@ __device__ __forceinline__ void group_segment(const Params& p, int64_t s, int64_
   const int64_t f0 = (int64_t)feature_lane * VEC;
   if (f0 < d) {
     // Rows past the segment re-read its last row (in cache) instead of
-    // branching around the load, so the eight loads issue back to back.
+    // branching around the load, so the loads issue back to back.
     auto rows = [&](auto&& body) {
-      for (int64_t r = start; r < end; r += 8) {
-        float x[8][VEC];
+      constexpr int U = MASK && VEC > 2 ? 4 : 8;
+      for (int64_t r = start; r < end; r += U) {
+        float x[U][VEC];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) load_input<T, VEC, MASK>(p, (r + u < end ? r + u : end - 1) * d + f0, x[u]);
+        for (int u = 0; u < U; ++u) load_input<T, VEC, MASK>(p, (r + u < end ? r + u : end - 1) * d + f0, x[u]);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
+        for (int u = 0; u < U; ++u) {
           if (r + u < end) body(r + u, x[u]);
         }
       }
