@@ -45,8 +45,14 @@ enum rg_index { RG_I32 = 0, RG_I64 = 1 };
  * rows (the caller's max_len says so): one worker launch takes the segments
  * in order, with no classification and no workspace. Any input is still
  * computed exactly; a longer segment only runs slower. Not available when
- * alone_rows or t_wave is 0. */
-enum rg_schedule { RG_CLASSIFIED = 0, RG_BLOCK_PER_SEGMENT = 1, RG_SHORT_SEGMENTS = 2 };
+ * alone_rows or t_wave is 0.
+ * RG_TILES (sum and max with scale 1, no debug visits, a row of at most 64
+ * lanes): equal tiles of the
+ * rows and segment ends, one wave each, whatever the lengths are; a second
+ * launch adds what crosses tiles (none for one tile; up to 16 tiles one
+ * workgroup does both). items_cap is then the number of tiles and part_rows
+ * the positions of a tile. */
+enum rg_schedule { RG_CLASSIFIED = 0, RG_BLOCK_PER_SEGMENT = 1, RG_SHORT_SEGMENTS = 2, RG_TILES = 3 };
 
 /* Kernel roles (a plan lists its launches in submission order). */
 enum rg_role {
@@ -54,8 +60,8 @@ enum rg_role {
   RG_ROLE_CLASSIFY = 1,
   RG_ROLE_WAVE = 2,            /* not launched: the wave class runs inside RG_ROLE_WORKER */
   RG_ROLE_BLOCK = 3,           /* not launched: the block class runs inside RG_ROLE_WORKER */
-  RG_ROLE_SPLIT_PARTIAL = 4,   /* not launched: split parts run inside RG_ROLE_WORKER */
-  RG_ROLE_SPLIT_COMBINE = 5,   /* not launched: the last part of a segment combines, inside RG_ROLE_WORKER */
+  RG_ROLE_SPLIT_PARTIAL = 4,   /* RG_TILES: the tiles (split parts of the others run inside RG_ROLE_WORKER) */
+  RG_ROLE_SPLIT_COMBINE = 5,   /* RG_TILES: segments that cross tiles (else inside RG_ROLE_WORKER) */
   RG_ROLE_SPLIT_NORMALIZE = 6, /* not launched: the classified worker normalises split parts */
   RG_ROLE_NAIVE = 7,           /* block-per-segment schedule */
   RG_ROLE_FUSED = 8,           /* softmax: register-resident worker over all block/split items, then the
@@ -109,7 +115,7 @@ typedef struct rg_plan {
   int32_t roles[RG_MAX_LAUNCHES];         /* rg_role of each launch */
   uint32_t grid[RG_MAX_LAUNCHES][3];
   uint32_t block[RG_MAX_LAUNCHES];
-  uint32_t lds_bytes[RG_MAX_LAUNCHES];    /* static LDS of each kernel */
+  uint32_t lds_bytes[RG_MAX_LAUNCHES];    /* static LDS of each kernel (RG_ROLE_SPLIT_PARTIAL: dynamic) */
   uint64_t workspace_bytes;               /* one allocation, buffers 256-B aligned */
   uint64_t buffer_offset[RG_WORKSPACE_BUFFERS];
   uint64_t buffer_bytes[RG_WORKSPACE_BUFFERS];

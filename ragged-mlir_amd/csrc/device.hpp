@@ -240,6 +240,11 @@ struct Params {
   int64_t min_len, max_len;  // checked-offsets hints, -1 when absent
   int32_t short_segments;  // worker: every segment in order as wave class (no queues)
   int64_t alone_rows;      // wave-class segments a lane / lane group reduces alone
+  int64_t tile_count;      // tile schedule: tiles (one wave each)
+  int64_t tile_items;      // positions of the row / segment-end axis per tile
+  int32_t tile_batch;      // rows a wave stages at once
+  int32_t tile_single;     // one workgroup holds every tile and folds what crosses them
+  int64_t marker_rows;     // positions a segment's end takes on that axis
 };
 
 // ---------------------------------------------------------------------------

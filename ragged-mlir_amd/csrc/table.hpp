@@ -8,6 +8,7 @@
 #include <type_traits>
 
 #include "fused.hpp"
+#include "tiles.hpp"
 #include "worker.hpp"
 
 namespace rg {
@@ -17,6 +18,8 @@ struct KernelSet {
   const void* worker;            // classified schedule: wave, block and split classes in one launch
   const void* fused;             // softmax, row mapping: register-resident worker
   const void* fused_f32;         // same, storing f32 logits (scale or mask on bf16 input)
+  const void* tiles;             // sum, max, row mapping: equal tiles of the input
+  const void* tiles_fold;        // sum, max: segments that cross tiles
   int vec;                       // elements per vector access
   bool flat;                     // flat mapping (D < vec)
   int rpt;                       // rows per thread of `fused` (0: no fused worker)
@@ -48,6 +51,18 @@ constexpr int fused_rpt() {
     return 0;
 }
 
+template <int OP, class T, class OFFT, int VEC, bool FLAT>
+constexpr const void* tiles_kernel() {
+  if constexpr (OP != OP_SOFTMAX && !FLAT) return (const void*)&k_tiles<OP, T, OFFT, VEC>;
+  else return nullptr;
+}
+
+template <int OP, class T>
+constexpr const void* tiles_fold_kernel() {
+  if constexpr (OP != OP_SOFTMAX) return (const void*)&k_tiles_fold<OP, T>;
+  else return nullptr;
+}
+
 // Geometry index: f32 -> 0:row1 1:row2 2:row4 3:flat4; bf16 -> 0:row1 1:row2 2:row4 3:row8 4:flat8.
 constexpr int kGeometries = 5;
 
@@ -68,6 +83,7 @@ const void* kernel_offsets_check(int offsets_dtype);
    (const void*)&rg::k_worker<OP, T, OFFT, VEC, FLAT, MASK>,                              \
    rg::fused_kernel<OP, T, OFFT, VEC, FLAT, MASK, std::is_same<T, float>::value>(),              \
    rg::fused_kernel<OP, T, OFFT, VEC, FLAT, MASK, true>(),                                       \
+   rg::tiles_kernel<OP, T, OFFT, VEC, FLAT>(), rg::tiles_fold_kernel<OP, T>(),                   \
    VEC, FLAT,                                                                                    \
    rg::fused_rpt<OP, T, VEC, FLAT, MASK, std::is_same<T, float>::value>(),                       \
    rg::fused_rpt<OP, T, VEC, FLAT, MASK, true>()}
@@ -76,7 +92,7 @@ const void* kernel_offsets_check(int offsets_dtype);
 #define RG_GEOMETRIES(OP, OFFT, MASK)                                                           \
   {{RG_SET(OP, float, OFFT, 1, false, MASK), RG_SET(OP, float, OFFT, 2, false, MASK),          \
     RG_SET(OP, float, OFFT, 4, false, MASK), RG_SET(OP, float, OFFT, 4, true, MASK),           \
-    {nullptr, nullptr, nullptr, nullptr, 0, false, 0, 0}},                                      \
+    {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, false, 0, 0}},                                      \
    {RG_SET(OP, __bf16, OFFT, 1, false, MASK), RG_SET(OP, __bf16, OFFT, 2, false, MASK),        \
     RG_SET(OP, __bf16, OFFT, 4, false, MASK), RG_SET(OP, __bf16, OFFT, 8, false, MASK),        \
     RG_SET(OP, __bf16, OFFT, 8, true, MASK)}}

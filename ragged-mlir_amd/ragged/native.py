@@ -21,7 +21,7 @@ ABI_VERSION = 3
 OPS = {"sum": 0, "max": 1, "softmax": 2}
 DTYPES = {"f32": 0, "bf16": 1}
 INDEX_DTYPES = {"i32": 0, "i64": 1}
-SCHEDULES = {"classified": 0, "naive": 1, "short": 2}
+SCHEDULES = {"classified": 0, "naive": 1, "short": 2, "tiles": 3}
 ROLES = ("init", "classify", "wave", "block", "split_partial", "split_combine", "split_normalize", "naive",
          "fused", "deferred", "worker")
 BUFFERS = ("class_counts", "segment_ids", "item_segments", "part_begin", "partials", "partial_sums",

@@ -214,6 +214,13 @@ class CompiledProgram:
         # Workspace per (device, stream): calls on one stream run in order,
         # so they can share it; it grows to the largest plan seen.
         self._workspaces: dict[tuple[int, int], Any] = {}
+        # Sum / max run as equal tiles when the schedule is the library's to
+        # choose (an adaptive program with every mapping on) and the tile
+        # kernels take the spec (no scale, a row of at most 64 lanes).
+        options = spec.optimizations
+        lanes = 1 if self._metadata["mapping"] == "flat" else -(-spec.feature_dim // self._metadata["d_vector"])
+        self._tiles = (spec.op != "softmax" and self._selects and float(self._metadata["scale"]) == 1.0
+                       and lanes <= 64 and options.warp_mapping and options.split_mapping)
         self._names = {kernel["role"]: kernel["name"] for kernel in self._metadata["kernels"]}
         self._alone: int | None = None
         self._wait_limit: dict[int, int] = {}   # device -> longest segment (rows) the register path holds
@@ -476,6 +483,11 @@ class CompiledProgram:
         if self.naive is not None and select != "classified":
             if select == "naive":
                 chosen, selection = "naive", {"forced": True}
+            elif self._tiles:
+                # Sum / max: equal tiles of the input, whatever the lengths.
+                return self._run(values, offsets, out, stream, mode, debug_buffers=debug_buffers, mask=mask,
+                                 selected="classified", selection={"max_len": max_len, "tiles": True},
+                                 schedule="tiles")
             elif self._short_segments(max_len):
                 # One worker launch reduces every segment alone: cheaper than
                 # both modelled schedules, so the model is not consulted.
@@ -492,7 +504,7 @@ class CompiledProgram:
                                  "reason": "segments too long to hold in registers carry at least half the rows "
                                            "and 1.5 register limits"}
                     return self._run(values, offsets, out, stream, mode, debug_buffers=debug_buffers, mask=mask,
-                                     selected="classified", selection=selection, max_len=max_len, streaming=True)
+                                     selected="classified", selection=selection, max_len=max_len, schedule="stream")
                 chosen, selection = (self.choose(n, b, max_len, device_l2_mib(values)) if n is not None
                                      else ("classified", {}))
             if chosen == "naive":
@@ -532,7 +544,7 @@ class CompiledProgram:
                 and 0 < self._alone_rows() and max_len <= self._alone_rows())
 
     def _run(self, values, offsets, out, stream, mode, *, debug_buffers, mask, selected, selection,
-             max_len: int | None = None, streaming: bool = False) -> ExecutionReport:
+             max_len: int | None = None, schedule: str | None = None) -> ExecutionReport:
         if mode not in ("validated", "checked"):
             raise ValidationError("mode must be validated or checked")
         if self.spec.mask != (mask is not None):
@@ -587,11 +599,13 @@ class CompiledProgram:
                 if b == 0:
                     return self._report(started, names, grids, 0, mode=mode, selected=selected, selection=selection,
                                         validation_bytes=validation_bytes, validation_ms=validation_ms)
-            short = not streaming and self._short_segments(max_len)
-            if short:
+            forced = schedule        # "tiles" or "stream", or the program's own
+            if forced is None and self._short_segments(max_len):
+                schedule = "short"
                 selection = {**selection, "short_segments": True}
-            schedule = "stream" if streaming else "short" if short else self._schedule
-            if streaming:
+            elif forced is None:
+                schedule = self._schedule
+            if forced == "stream":
                 module = self._stream_module(device)
             elif schedule == "classified" and self.spec.op != "softmax" and not self.spec.debug_visits:
                 default_rows = int(self._metadata["part_rows"])

@@ -1,0 +1,87 @@
+"""The tile schedule of sum and max (csrc/tiles.hpp) against the oracle, at the
+sizes where it can go wrong: one tile, one workgroup of tiles, many tiles;
+segments inside a batch of a wave (several at once from LDS, and longer ones
+among them), across batches, across tiles and over more tiles than one lane
+folds; empty segments at both ends and between; array ends inside a vector;
+every access width, the flat mapping and the widest rows (64 lanes)."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from ragged import Compiler, Optimizations, ProgramSpec
+from ragged.workloads import offsets_from_lengths
+
+pytestmark = pytest.mark.gpu
+
+GEOMETRIES = [("f32", 1), ("f32", 2), ("f32", 3), ("f32", 4), ("f32", 6), ("f32", 16), ("f32", 25), ("f32", 128),
+              ("f32", 256), ("bf16", 1), ("bf16", 2), ("bf16", 4), ("bf16", 5), ("bf16", 8),
+              ("bf16", 84), ("bf16", 128), ("bf16", 512)]
+
+
+def lengths_of(kind, d, elements):
+    """Lengths of about ``elements`` values in all."""
+    rng = np.random.default_rng(len(kind) * 1000 + d)
+    rows = max(6, elements // d)
+    if kind == "tiny":              # zero to three rows, empty runs at both ends
+        lengths = rng.integers(0, 4, max(8, rows // 2))
+        lengths[:5] = lengths[-70:] = 0
+    elif kind == "middle":          # around a batch of a wave
+        lengths = rng.integers(1, max(2, 2 * (1024 // d) + 3), max(3, rows // (1024 // d + 2)))
+    elif kind == "spread":          # one long segment in sixteen among short ones
+        lengths = np.where(np.arange(max(8, rows // 40)) % 16 == 7, 600 // min(d, 32) + 17, rng.integers(1, 6))
+    else:                           # one segment holds nearly everything
+        lengths = np.array([3, 0, rows + 1, 1, 0])
+    return lengths.astype(np.int64)
+
+
+@pytest.mark.parametrize("dtype,d", GEOMETRIES)
+@pytest.mark.parametrize("op", ["sum", "max"])
+def test_tiles_match_the_oracle(artifact_cache, op, dtype, d):
+    from gpu_helpers import check, run_program
+    offsets_dtype = "i32" if d % 2 else "i64"
+    program = Compiler().compile(ProgramSpec(op, dtype, d, offsets_dtype), artifact_cache)
+    launches = set()
+    for elements in (700, 40_000, 900_000):
+        for kind in ("tiny", "middle", "spread", "one"):
+            offsets = offsets_from_lengths(lengths_of(kind, d, elements), offsets_dtype)
+            values = np.random.default_rng(7).normal(size=(int(offsets[-1]), d)).astype(np.float32)
+            print(op, dtype, d, kind, values.shape, len(offsets) - 1, flush=True)
+            actual, report = run_program(program, values, offsets, dtype=dtype, op=op)
+            assert report.selection.get("tiles") and report.kernel_names[0].endswith("split_partial")
+            launches.add(len(report.kernel_names))
+            check(actual, values, offsets, op=op, dtype=dtype)
+    assert launches == {1, 2}       # one workgroup, and tiles folded by a second launch
+
+
+@pytest.mark.parametrize("op,dtype,d", [("sum", "f32", 1), ("max", "bf16", 5), ("sum", "bf16", 16)])
+def test_tiles_element_access(artifact_cache, op, dtype, d):
+    """One element per access (unaligned views), non-finite values."""
+    from gpu_helpers import check, run_program
+    program = Compiler().compile(ProgramSpec(op, dtype, d, "i64", optimizations=Optimizations(vectorize=False)),
+                                 artifact_cache)
+    rng = np.random.default_rng(3)
+    offsets = offsets_from_lengths(rng.integers(0, 90, 900).astype(np.int64), "i64")
+    values = rng.normal(size=(int(offsets[-1]), d)).astype(np.float32)
+    values[rng.random(values.shape) < 0.003] = np.nan
+    values[rng.random(values.shape) < 0.003] = -np.inf
+    actual, report = run_program(program, values, offsets, dtype=dtype, op=op)
+    assert report.selection.get("tiles")
+    check(actual, values, offsets, op=op, dtype=dtype)
+
+
+@pytest.mark.parametrize("op,dtype,d", [("sum", "f32", 2), ("sum", "bf16", 128), ("max", "f32", 100)])
+def test_tiles_repeat_bit_for_bit_and_share_a_workspace(artifact_cache, op, dtype, d):
+    """The chains' order does not depend on scheduling, and a call on the
+    classified schedule between (same workspace) changes nothing."""
+    from gpu_helpers import run_program
+    program = Compiler().compile(ProgramSpec(op, dtype, d, "i64"), artifact_cache)
+    rng = np.random.default_rng(11)
+    lengths = np.concatenate([[300_000 // d], rng.integers(0, 300, 2000)]).astype(np.int64)
+    offsets = offsets_from_lengths(lengths, "i64")
+    values = rng.normal(size=(int(offsets[-1]), d)).astype(np.float32)
+    first, _ = run_program(program, values, offsets, dtype=dtype, op=op)
+    classified, _ = run_program(program, values, offsets, dtype=dtype, op=op, select="classified")
+    again, _ = run_program(program, values, offsets, dtype=dtype, op=op)
+    classified_again, _ = run_program(program, values, offsets, dtype=dtype, op=op, select="classified")
+    assert np.array_equal(first, again) and np.array_equal(classified, classified_again)
