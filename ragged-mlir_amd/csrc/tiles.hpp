@@ -36,10 +36,11 @@ constexpr int kTileLoads = kTileStage / (kWave * 16);
 constexpr int kTileAux = kStreamAux;
 constexpr int kTileThreads = 1024;    // largest workgroup of k_tiles
 constexpr int kFoldFlight = 8;        // k_tiles_fold: partials in flight per lane
-constexpr int kFoldParts = 16;        // k_tiles_fold: longest chain one lane per feature folds
+constexpr int kFoldParts = 32;        // k_tiles_fold: longest chain one lane per feature folds
+constexpr int kFoldWave = 64;         // k_tiles_fold: parts per lane up to which a wave folds a chain
 constexpr int kFoldFeatures = 16;     // k_tiles_fold: features per workgroup
-constexpr int kTileFoldBytes = 4 * (kTileThreads + 32);   // LDS of a fold: one float per thread and the list
-constexpr int kFoldLong = 16;         // k_tiles_fold: longer chains one workgroup can meet (kBlock / kFoldParts)
+constexpr int kFoldLong = kTileThreads / kFoldParts;      // longer chains one workgroup's tiles can end
+constexpr int kTileFoldBytes = 4 * (kTileThreads + kFoldLong + 1);   // LDS of a fold: a float per thread, the list
 constexpr int kGroupSteps = 32;       // rows per lane up to which segments of a batch are reduced side by side
 
 // Lanes per tile in k_tiles_fold: a power of two, at most kFoldFeatures.
@@ -180,25 +181,44 @@ __device__ __forceinline__ void fold_tiles(const Params& p, int64_t tile0, int l
     }
   }
   __syncthreads();
+  // Longer chains: a wave each, its lanes on contiguous runs of parts; those
+  // too long for a wave the whole workgroup.
   const int many = *list < kFoldLong ? *list : kFoldLong;
-  const int pl = t / lanes, pl_count = threads / lanes;
-  for (int k = 0; k < many; ++k) {
-    const int64_t w2 = tile0 + list[1 + k];
-    const int64_t s2 = p.item_pos[w2], first2 = first_of(w2), count = w2 - first2;
-    State<OP> acc;
+  const int in_wave = kWave / lanes;
+  auto shared = [&](State<OP>& acc, int k, int pl, int pl_count) {
+    const int64_t w2 = tile0 + list[1 + k], first2 = first_of(w2), count = w2 - first2;
     acc.init();
     if (f < d) add_tails(acc, first2 + count * pl / pl_count, first2 + count * (pl + 1) / pl_count);
+  };
+  auto parts_of = [&](int k) { return tile0 + list[1 + k] - first_of(tile0 + list[1 + k]); };
+  auto finish = [&](State<OP>& acc, int k) {
+    const int64_t w2 = tile0 + list[1 + k];
+    add(acc, part[w2 * 2 * d + f]);
+    Elem<T>::put(out + p.item_pos[w2] * d + f, exact_value<OP>(acc));
+  };
+  for (int k = t / kWave; k < many; k += threads / kWave) {
+    if (parts_of(k) > kFoldWave * in_wave) continue;
+    State<OP> acc;
+    shared(acc, k, (t & (kWave - 1)) / lanes, in_wave);
+    xor_butterfly_range(lanes, kWave, [&](auto mask) {
+      merge_exact<OP>(acc, shfl_xor_exact<decltype(mask)::value, OP>(acc));
+    });
+    if ((t & (kWave - 1)) < lanes && f < d) finish(acc, k);
+  }
+  for (int k = 0; k < many; ++k) {
+    if (parts_of(k) <= kFoldWave * in_wave) continue;
+    State<OP> acc;
+    shared(acc, k, t / lanes, threads / lanes);
     __syncthreads();
     lds[t] = exact_value<OP>(acc);
     __syncthreads();
-    if (pl == 0 && f < d) {
-      State<OP> all;
-      all.init();
-      for (int q = 0; q < pl_count; ++q) add(all, lds[q * lanes + fl]);
-      add(all, part[w2 * 2 * d + f]);
-      Elem<T>::put(out + s2 * d + f, exact_value<OP>(all));
+    if (t < lanes && f < d) {
+      acc.init();
+      for (int q = 0; q < threads / lanes; ++q) add(acc, lds[q * lanes + fl]);
+      finish(acc, k);
     }
   }
+  __syncthreads();      // before the list is used again
 }
 
 // A call's partials overlap what a register-resident softmax plan keeps at
@@ -434,7 +454,10 @@ __global__ __launch_bounds__(kTileThreads) void k_tiles(Params p) {
   }
   if (p.tile_single) {
     // One workgroup holds every tile: it folds the chains itself, in the
-    // staging memory, which no wave uses any more.
+    // staging memory, which no wave uses any more. (Doing this for more
+    // workgroups, the last one out folding, took 11.4 us where the two
+    // launches take 7.8 and 8.8: the release, the count and the fold follow
+    // one another.)
     __threadfence_block();
     __syncthreads();
     float* lds = reinterpret_cast<float*>(tile_lds);
