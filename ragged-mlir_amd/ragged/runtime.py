@@ -210,7 +210,7 @@ class CompiledProgram:
         self._plans: dict[tuple[native.NativeModule, int, int, str], native.Plan] = {}
         # Per plan: its kernel names and grids for reports, and the ctypes
         # reference rg_run takes (built once, not per call).
-        self._launches: dict[tuple[native.NativeModule, int, int, str], tuple[list, list, Any]] = {}
+        self._launches: dict[tuple[native.NativeModule, int, int, str], tuple[tuple, tuple, Any]] = {}
         # Workspace per (device, stream): calls on one stream run in order,
         # so they can share it; it grows to the largest plan seen.
         self._workspaces: dict[tuple[int, int], Any] = {}
@@ -224,8 +224,9 @@ class CompiledProgram:
         self._names = {kernel["role"]: kernel["name"] for kernel in self._metadata["kernels"]}
         self._alone: int | None = None
         self._wait_limit: dict[int, int] = {}   # device -> longest segment (rows) the register path holds
+        self._facts: tuple | None = None    # what _tensor_facts compares with
         self._torch_dtypes: tuple | None = None    # (values dtype, offsets dtype) as torch dtypes
-        self._report_static: tuple | None = None   # (classes, thresholds) of every report
+        self._report_template: dict | None = None  # the fields every report shares
 
     @property
     def selects(self) -> bool:
@@ -349,6 +350,114 @@ class CompiledProgram:
             raise ValidationError("in-place specialization requires out and values to be the same buffer")
         return n, b
 
+    def _tensor_facts(self, torch, values, offsets, out, mask):
+        """(n, b, device, three data pointers, mask pointer) of a call that
+        passes ``_validate_tensors`` -- the same conditions, each tensor
+        property read once -- or None for anything else: empty tensors, a
+        Tensor subclass, or a call that method refuses and explains."""
+        tensor = torch.Tensor
+        if type(values) is not tensor or type(offsets) is not tensor or type(out) is not tensor:
+            return None
+        facts = self._facts
+        if facts is None:
+            metadata, spec = self._metadata, self.spec
+            vector, element = metadata["d_vector"], 2 if spec.dtype == "bf16" else 4
+            wide = min(16, vector * element) - 1 if vector > 1 else 0
+            scalar_out = spec.op != "softmax" and metadata["mapping"] == "flat"
+            facts = self._facts = (
+                {"f32": torch.float32, "bf16": torch.bfloat16}[spec.dtype],
+                {"i32": torch.int32, "i64": torch.int64}[spec.offsets_dtype],
+                spec.feature_dim, spec.feature_dim * element, 4 if spec.offsets_dtype == "i32" else 8, wide,
+                0 if scalar_out else wide, min(16, vector * 4) - 1 if vector > 1 else 0,
+                spec.op == "softmax", spec.alias == "inplace",
+                2**31 - 1 if spec.offsets_dtype == "i32" else I64_MAX, torch.float32)
+        dtype, offset_dtype, d, row, offset_bytes, wide, out_wide, mask_wide, softmax, inplace, most, f32 = facts
+        device = values.get_device()
+        if (device < 0 or offsets.get_device() != device or out.get_device() != device
+                or values.dtype != dtype or offsets.dtype != offset_dtype or out.dtype != dtype
+                or not values.is_contiguous() or not offsets.is_contiguous() or not out.is_contiguous()
+                or values.requires_grad or offsets.requires_grad or out.requires_grad):
+            return None
+        shape, ends, result = values.shape, offsets.shape, out.shape
+        if len(shape) != 2 or shape[1] != d or len(ends) != 1 or len(result) != 2 or result[1] != d:
+            return None
+        n, b = shape[0], ends[0] - 1
+        rows = n if softmax else b
+        if n < 1 or b < 1 or n > most or result[0] != rows:
+            return None
+        v0, f0, o0 = values.data_ptr(), offsets.data_ptr(), out.data_ptr()
+        if v0 & wide or o0 & out_wide:
+            return None
+        v1, f1, o1 = v0 + n * row, f0 + (b + 1) * offset_bytes, o0 + rows * row
+        if (f0 < v1 and v0 < f1) or (f0 < o1 and o0 < f1):
+            return None
+        if v0 < o1 and o0 < v1:
+            if not (inplace and v0 == o0 and softmax):
+                return None
+        elif inplace:
+            return None
+        m0 = None
+        if mask is not None:
+            if (type(mask) is not tensor or mask.get_device() != device or mask.dtype != f32
+                    or not mask.is_contiguous() or mask.requires_grad or mask.shape != shape):
+                return None
+            m0 = mask.data_ptr()
+            m1 = m0 + n * d * 4
+            if m0 & mask_wide or (m0 < o1 and o0 < m1) or (m0 < f1 and f0 < m1):
+                return None
+        return n, b, device, v0, f0, o0, m0
+
+    def _quick(self, values, offsets, out, stream, mask, selected, selection, max_len, schedule):
+        """A validated call whose module, device and stream are known from an
+        earlier one: the work of ``_run`` without its general cases (it
+        returns None for those)."""
+        torch = _torch_module
+        if torch is None:
+            return None
+        facts = self._tensor_facts(torch, values, offsets, out, mask)
+        if facts is None:
+            return None
+        n, b, device, v0, f0, o0, m0 = facts
+        started = time.perf_counter()
+        module = _modules.get((device, self._digest))
+        if (module is None or device != torch._C._cuda_getDevice()
+                or not _device_runs.get((device, self.spec.chip))):
+            return None
+        if schedule is None:
+            if self._schedule == "classified" and self.spec.op != "softmax":
+                return None
+            schedule = self._schedule
+            if self._short_segments(max_len):
+                schedule = "short"
+                selection = {**selection, "short_segments": True}
+        elif schedule != "tiles":
+            return None
+        if stream is None:
+            active = _current_stream(torch, device)
+        elif isinstance(stream, torch.cuda.Stream) and stream.device_index == device:
+            active = stream
+        else:
+            return None
+        handle = active.cuda_stream
+        plan, names, grids, plan_ref = self._plan_launches(module, n, b, schedule)
+        nbytes, workspace = plan.workspace_bytes, None
+        if nbytes:
+            workspace = self._workspaces.get((device, handle))
+            if workspace is None or workspace.numel() < nbytes:
+                workspace = self._workspace(torch, values.device, active, nbytes, fresh=False)
+        values.record_stream(active)
+        offsets.record_stream(active)
+        out.record_stream(active)
+        if mask is not None:
+            mask.record_stream(active)
+        try:
+            module.run_ref(plan_ref, v0, f0, o0, m0, workspace.data_ptr() if nbytes else None, nbytes, handle)
+        except Exception:
+            # As in _run: the next call on this stream gets a fresh workspace.
+            self._workspaces.pop((device, handle), None)
+            raise
+        return self._report(started, names, grids, nbytes, mode="validated", selected=selected, selection=selection)
+
     def _module(self, device: int) -> native.NativeModule:
         key = (device, self._digest)
         module = _modules.get(key)
@@ -458,8 +567,8 @@ class CompiledProgram:
         launches = self._launches.get(key)
         if launches is None:
             steps = plan.steps
-            launches = self._launches[key] = ([self._kernel_name(role) for role, _, _, _ in steps],
-                                              [grid for _, grid, _, _ in steps], native.plan_ref(plan))
+            launches = self._launches[key] = (tuple(self._kernel_name(role) for role, _, _, _ in steps),
+                                              tuple(grid for _, grid, _, _ in steps), native.plan_ref(plan))
         return (plan,) + launches
 
     # ------------------------------------------------------------------
@@ -517,21 +626,34 @@ class CompiledProgram:
 
     def _report(self, started, plan_names=(), grids=(), workspace=0, *, mode, selected, selection,
                 validation_bytes=0, validation_ms=None) -> ExecutionReport:
-        metadata = self._metadata
-        static = self._report_static
-        if static is None:
-            static = self._report_static = (tuple(metadata["classes"]), tuple(metadata["thresholds"]))
-        thresholds = static[1]
+        template = self._report_template
+        if template is None:
+            metadata = self._metadata
+            template = self._report_template = dict(vars(ExecutionReport(
+                tuple(metadata["classes"]), tuple(metadata["thresholds"]), (), 0, self._digest,
+                cache_hit=self.cache_hit, optimizations=metadata["optimizations"], d_tile=metadata["d_tile"],
+                d_vector=metadata["d_vector"], streams=1)))
+        # The frozen record's fields, set at once (its __init__ sets each
+        # through object.__setattr__: 1.6 us a call).
+        report = object.__new__(ExecutionReport)
+        fields = vars(report)
+        fields.update(template)
+        if not plan_names:
+            fields["classes"] = ()
         if selection and "t_block" in selection:
             # A companion module's block threshold (big_block_rows).
-            thresholds = (thresholds[0], selection["t_block"]) + thresholds[2:]
-        return ExecutionReport(
-            static[0] if plan_names else (), thresholds, tuple(grids),
-            workspace + validation_bytes, self._digest, None, mode, tuple(plan_names),
-            (time.perf_counter() - started) * 1000, cache_hit=self.cache_hit,
-            validation_workspace_bytes=validation_bytes, validation_host_ms=validation_ms,
-            optimizations=metadata["optimizations"], d_tile=metadata["d_tile"], d_vector=metadata["d_vector"],
-            resources=None, streams=1, selected=selected, selection=selection)
+            thresholds = template["thresholds"]
+            fields["thresholds"] = (thresholds[0], selection["t_block"]) + thresholds[2:]
+        fields["grids"] = tuple(grids)
+        fields["workspace_bytes"] = workspace + validation_bytes
+        fields["mode"] = mode
+        fields["kernel_names"] = tuple(plan_names)
+        fields["host_enqueue_ms"] = (time.perf_counter() - started) * 1000
+        fields["validation_workspace_bytes"] = validation_bytes
+        fields["validation_host_ms"] = validation_ms
+        fields["selected"] = selected
+        fields["selection"] = selection
+        return report
 
     def _short_segments(self, max_len: int | None) -> bool:
         """Whether the caller's max_len lets one lane (or lane group) reduce
@@ -545,6 +667,11 @@ class CompiledProgram:
 
     def _run(self, values, offsets, out, stream, mode, *, debug_buffers, mask, selected, selection,
              max_len: int | None = None, schedule: str | None = None) -> ExecutionReport:
+        if mode == "validated" and debug_buffers is None and not self.spec.debug_visits \
+                and self.spec.mask == (mask is not None):
+            report = self._quick(values, offsets, out, stream, mask, selected, selection, max_len, schedule)
+            if report is not None:
+                return report
         if mode not in ("validated", "checked"):
             raise ValidationError("mode must be validated or checked")
         if self.spec.mask != (mask is not None):
