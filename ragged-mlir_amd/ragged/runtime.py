@@ -125,6 +125,26 @@ def big_block_rows(n: int, part_rows: int, default_t_block: int) -> int:
     return max(default_t_block, min(part_rows, n // BIG_BLOCK_SHARE // step * step))
 
 
+# Small sum / max calls whose longest segment is provably short enough for
+# one workgroup run block per segment: one launch and no search, where the
+# tiles' two cost the host 3.3 us and a round trip more (8.7 against 10.5-12
+# us per call, 19 against 24 us alone). Measured over 64 KiB-16 MiB and 1-8,192
+# segments: up to 8 KiB of rows per byte of access width (f32 D=128 128 KiB, f32
+# D=25 32 KiB, bf16 D=5 16 KiB) block per segment is as fast or faster, twice
+# that is the break-even; 8,192 segments break even too.
+SMALL_CALL_BYTES = 16 << 20
+SMALL_LONGEST_PER_ACCESS = 8 << 10
+SMALL_SEGMENTS = 4096
+
+
+def small_reduce(n: int, b: int, max_len: int | None, row_bytes: int, access_bytes: int) -> bool:
+    """Whether a sum / max call of (n, b) rows and segments, its longest
+    segment at most ``max_len`` (None: n) rows, runs block per segment."""
+    longest = n if max_len is None else min(max_len, n)
+    return (b <= SMALL_SEGMENTS and n * row_bytes <= SMALL_CALL_BYTES
+            and longest * row_bytes <= SMALL_LONGEST_PER_ACCESS * access_bytes)
+
+
 def splits_segments(n: int, b: int, max_len: int | None, t_block: int) -> bool:
     """Whether a call of (n, b, max_len) provably holds a segment longer than
     the block class (``t_block`` rows): by max_len, or else by more rows than
@@ -218,6 +238,8 @@ class CompiledProgram:
         # choose (an adaptive program with every mapping on) and the tile
         # kernels take the spec (no scale, a row of at most 64 lanes).
         options = spec.optimizations
+        self._row_bytes = spec.feature_dim * (2 if spec.dtype == "bf16" else 4)
+        self._access_bytes = self._metadata["d_vector"] * (2 if spec.dtype == "bf16" else 4)
         lanes = 1 if self._metadata["mapping"] == "flat" else -(-spec.feature_dim // self._metadata["d_vector"])
         self._tiles = (spec.op != "softmax" and self._selects and float(self._metadata["scale"]) == 1.0
                        and lanes <= 64 and options.warp_mapping and options.split_mapping)
@@ -593,10 +615,18 @@ class CompiledProgram:
             if select == "naive":
                 chosen, selection = "naive", {"forced": True}
             elif self._tiles:
-                # Sum / max: equal tiles of the input, whatever the lengths.
-                return self._run(values, offsets, out, stream, mode, debug_buffers=debug_buffers, mask=mask,
-                                 selected="classified", selection={"max_len": max_len, "tiles": True},
-                                 schedule="tiles")
+                # Sum / max: one workgroup per segment for small calls, else
+                # equal tiles of the input, whatever the lengths.
+                try:
+                    small = small_reduce(values.shape[0], offsets.shape[0] - 1, max_len, self._row_bytes,
+                                         self._access_bytes)
+                except (AttributeError, IndexError, TypeError):
+                    small = False       # not tensors: validation reports it
+                if not small:
+                    return self._run(values, offsets, out, stream, mode, debug_buffers=debug_buffers, mask=mask,
+                                     selected="classified", selection={"max_len": max_len, "tiles": True},
+                                     schedule="tiles")
+                chosen, selection = "naive", {"max_len": max_len, "reason": "small call, short segments"}
             elif self._short_segments(max_len):
                 # One worker launch reduces every segment alone: cheaper than
                 # both modelled schedules, so the model is not consulted.

@@ -9,6 +9,7 @@ import pytest
 
 torch = pytest.importorskip("torch")
 
+from ragged import runtime
 from ragged import Compiler, Optimizations, ProgramSpec
 from ragged.workloads import offsets_from_lengths
 
@@ -37,11 +38,12 @@ def lengths_of(kind, d, elements):
 
 @pytest.mark.parametrize("dtype,d", GEOMETRIES)
 @pytest.mark.parametrize("op", ["sum", "max"])
-def test_tiles_match_the_oracle(artifact_cache, op, dtype, d):
+def test_tiles_match_the_oracle(artifact_cache, monkeypatch, op, dtype, d):
     from gpu_helpers import check, run_program
     offsets_dtype = "i32" if d % 2 else "i64"
     program = Compiler().compile(ProgramSpec(op, dtype, d, offsets_dtype), artifact_cache)
     launches = set()
+    monkeypatch.setattr(runtime, "SMALL_SEGMENTS", 0)      # small calls too
     for elements in (700, 40_000, 900_000):
         for kind in ("tiny", "middle", "spread", "one"):
             offsets = offsets_from_lengths(lengths_of(kind, d, elements), offsets_dtype)
@@ -85,3 +87,23 @@ def test_tiles_repeat_bit_for_bit_and_share_a_workspace(artifact_cache, op, dtyp
     again, _ = run_program(program, values, offsets, dtype=dtype, op=op)
     classified_again, _ = run_program(program, values, offsets, dtype=dtype, op=op, select="classified")
     assert np.array_equal(first, again) and np.array_equal(classified, classified_again)
+
+
+@pytest.mark.parametrize("op,dtype,d", [("sum", "f32", 1), ("max", "bf16", 5)])
+def test_small_calls_run_block_per_segment(artifact_cache, op, dtype, d):
+    """A call that fits the small rule is one launch; one segment more, one
+    row more or an unknown longest segment beyond it is not."""
+    from gpu_helpers import check, run_program
+    program = Compiler().compile(ProgramSpec(op, dtype, d, "i32"), artifact_cache)
+    row = d * (2 if dtype == "bf16" else 4)
+    most = runtime.SMALL_LONGEST_PER_ACCESS * (16 if d == 1 else 2) // row       # rows of the longest segment
+    rng = np.random.default_rng(2)
+    for lengths, max_len, small in (([most, 0, 3], most, True), ([most, 0, 3], None, False), ([most - 3, 0, 3], None, True),
+                                    ([most + 1, 5], most + 1, False), ([2] * runtime.SMALL_SEGMENTS, 2, True),
+                                    ([2] * (runtime.SMALL_SEGMENTS + 1), 2, False)):
+        offsets = offsets_from_lengths(np.array(lengths, dtype=np.int64), "i32")
+        values = rng.normal(size=(int(offsets[-1]), d)).astype(np.float32)
+        actual, report = run_program(program, values, offsets, dtype=dtype, op=op, max_len=max_len)
+        assert report.selected == ("naive" if small else "classified")
+        assert bool(report.selection.get("tiles")) != small
+        check(actual, values, offsets, op=op, dtype=dtype)
