@@ -59,7 +59,8 @@ enum rg_role {
   RG_ROLE_INIT = 0,            /* not launched: k_classify initialises what a call uses */
   RG_ROLE_CLASSIFY = 1,
   RG_ROLE_WAVE = 2,            /* not launched: the wave class runs inside RG_ROLE_WORKER */
-  RG_ROLE_BLOCK = 3,           /* not launched: the block class runs inside RG_ROLE_WORKER */
+  RG_ROLE_BLOCK = 3,           /* block-per-segment softmax that holds segments in registers (the block class
+                                  of the classified schedule runs inside RG_ROLE_WORKER) */
   RG_ROLE_SPLIT_PARTIAL = 4,   /* RG_TILES: the tiles (split parts of the others run inside RG_ROLE_WORKER) */
   RG_ROLE_SPLIT_COMBINE = 5,   /* RG_TILES: segments that cross tiles (else inside RG_ROLE_WORKER) */
   RG_ROLE_SPLIT_NORMALIZE = 6, /* not launched: the classified worker normalises split parts */

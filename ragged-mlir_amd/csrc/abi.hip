@@ -67,6 +67,13 @@ constexpr int64_t kTileWavesPerCu = 12;
 constexpr int64_t kMarkerBytes = 256;
 constexpr int64_t kTileMaxBytes = 1 << 30;  // 32-bit offsets inside a tile
 
+// Block-per-segment softmax: up to this mean segment the kernel that holds
+// segments in registers (16 rows of 16 bytes per thread, half of that flat).
+// Measured per call, streaming -> held: bf16 D=64 41 KB longest 13.8 -> 9.1 us, 12
+// KB 36.1 -> 23.8; f32 D=1 10 KB 12.0 -> 8.2; bf16 D=1 100 B 180 -> 82; but 488
+// KB (bf16 D=128) 157 -> 174: streaming wants more workgroups per CU.
+constexpr int64_t kHeldBytes = 64 << 10;
+
 int element_bytes(int dtype) { return dtype == RG_BF16 ? 2 : 4; }
 
 // Geometry of a specialisation: elements per access and mapping, plus the
@@ -340,6 +347,7 @@ int rg_module_create(int device, const rg_spec* spec_in, rg_module** out) {
   module->roles[RG_ROLE_WORKER] = k.worker;
   // RG_ROLE_SPLIT_NORMALIZE stays empty: k_worker normalises split parts.
   module->roles[RG_ROLE_NAIVE] = k.naive;
+  module->roles[RG_ROLE_BLOCK] = k.naive_held;
   if (spec.op != RG_OP_SOFTMAX && feature_tiles(spec.feature_dim, module->geometry.vec, module->geometry.flat, rg::kWave) == 1) {
     // A narrow feature dimension (flat mapping elsewhere) is a row of one
     // D-element lane here.
@@ -599,7 +607,10 @@ int rg_plan_create(const rg_module* module, int64_t n, int64_t b, int schedule, 
   };
   const int64_t tiles_block = feature_tiles(d, geo.vec, geo.flat, rg::kBlock);
   if (schedule == RG_BLOCK_PER_SEGMENT) {
-    add_launch(RG_ROLE_NAIVE, b, tiles_block);
+    // A softmax whose mean segment a workgroup can hold holds them.
+    const bool held = module->roles[RG_ROLE_BLOCK] &&
+                      n <= b * ((geo.flat ? kHeldBytes / 2 : kHeldBytes) / (d * (int64_t)element_bytes(spec.dtype)));
+    add_launch(held ? RG_ROLE_BLOCK : RG_ROLE_NAIVE, b, tiles_block);
     return RG_OK;
   }
   if (schedule == RG_SHORT_SEGMENTS) {

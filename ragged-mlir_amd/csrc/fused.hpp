@@ -170,81 +170,6 @@ __device__ __forceinline__ void buffer_store(Rsrc r, int voffset, int soffset, c
   }
 }
 
-// VEC elements of S as 32-bit words: unpack to f32 / pack from f32.
-template <class S, int VEC> struct Words {
-  static constexpr int kBytes = VEC * (int)sizeof(S);
-  static constexpr int kCount = kBytes >= 4 ? kBytes / 4 : 1;
-  __device__ static float get(const uint32_t* w, int i) {
-    if constexpr (sizeof(S) == 4) return __uint_as_float(w[i]);
-    else return (i & 1) ? bf16_hi(w[i >> 1]) : bf16_lo(w[i >> 1]);
-  }
-  __device__ static void set(uint32_t* w, const float (&x)[VEC]) {
-    if constexpr (sizeof(S) == 4) {
-#pragma unroll
-      for (int i = 0; i < VEC; ++i) w[i] = __float_as_uint(x[i]);
-    } else if constexpr (VEC == 1) {
-      w[0] = pack_bf16(x[0], 0.f) & 0xffffu;
-    } else {
-#pragma unroll
-      for (int i = 0; i < kCount; ++i) w[i] = pack_bf16(x[2 * i], x[2 * i + 1]);
-    }
-  }
-  // -inf in every element (identity of the column max, zero mass).
-  __device__ static void fill_neg_inf(uint32_t* w) {
-#pragma unroll
-    for (int i = 0; i < kCount; ++i) w[i] = sizeof(S) == 4 ? 0xff800000u : 0xff80ff80u;
-  }
-};
-
-// Column reduction over the lanes of a workgroup that share a feature lane
-// (ROW mapping, lpr lanes per row): xor butterfly within each wave, then one
-// LDS pass across the four waves. Every thread receives its features' total.
-template <bool MAX, int VEC>
-__device__ __forceinline__ void block_allreduce(float (&v)[VEC], int lpr, int feat_lane, float* lds) {
-  const int t = threadIdx.x, lane = t & (kWave - 1), w = t / kWave;
-  auto combine = [](float a, float b) { return MAX ? fmax_nan(a, b) : a + b; };
-  xor_butterfly(lpr, [&](auto mask) {
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) v[i] = combine(v[i], xor_lane<decltype(mask)::value>(v[i]));
-  });
-  const int rep = lpr < kWave ? lpr : kWave;
-  if (lane < rep) {
-    float* slot = lds + (w * kWave + lane) * VEC;
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) slot[i] = v[i];
-  }
-  __syncthreads();
-  if (lpr <= kWave) {
-    // Every wave holds every feature lane: fold waves 0..3 in order, at
-    // fixed offsets from one base address.
-    const float* base = lds + feat_lane * VEC;
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) {
-      float acc = base[i];
-#pragma unroll
-      for (int ww = 1; ww < kWavesPerBlock; ++ww) acc = combine(acc, base[ww * kWave * VEC + i]);
-      v[i] = acc;
-    }
-  } else {
-    // A row spans lpr / 64 waves: feature lane fl lives in every
-    // (lpr/64)-th wave starting at fl / 64.
-    const int stride = lpr / kWave;
-    // Opaque: keeps the compiler from precomputing (and spilling) these
-    // addresses across the caller's loop for this rarely taken branch.
-    int offset = ((feat_lane / kWave) * kWave + (feat_lane & (kWave - 1))) * VEC;
-    asm volatile("" : "+v"(offset));
-    const float* base = lds + offset;
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) {
-      float acc = base[i];
-      for (int ww = feat_lane / kWave + stride; ww < kWavesPerBlock; ww += stride)
-        acc = combine(acc, base[(ww - feat_lane / kWave) * kWave * VEC + i]);
-      v[i] = acc;
-    }
-  }
-  __syncthreads();
-}
-
 // Statistics shared between workgroups travel only through agent-scope
 // atomic stores and loads (coherent across the XCDs' L2 caches), so no
 // L2-wide writeback or invalidate is needed. Each (m, s) pair of a feature is

@@ -8,6 +8,7 @@
 #include <type_traits>
 
 #include "fused.hpp"
+#include "held.hpp"
 #include "tiles.hpp"
 #include "worker.hpp"
 
@@ -15,6 +16,7 @@ namespace rg {
 
 struct KernelSet {
   const void* naive;
+  const void* naive_held;        // softmax without a mask: the same, holding segments in registers
   const void* worker;            // classified schedule: wave, block and split classes in one launch
   const void* fused;             // softmax, row mapping: register-resident worker
   const void* fused_f32;         // same, storing f32 logits (scale or mask on bf16 input)
@@ -63,6 +65,12 @@ constexpr const void* tiles_fold_kernel() {
   else return nullptr;
 }
 
+template <int OP, class T, class OFFT, int VEC, bool FLAT, bool MASK>
+constexpr const void* naive_held_kernel() {
+  if constexpr (OP == OP_SOFTMAX && !MASK) return (const void*)&k_naive<OP, T, OFFT, VEC, FLAT, false, true>;
+  else return nullptr;
+}
+
 // Geometry index: f32 -> 0:row1 1:row2 2:row4 3:flat4; bf16 -> 0:row1 1:row2 2:row4 3:row8 4:flat8.
 constexpr int kGeometries = 5;
 
@@ -80,6 +88,7 @@ const void* kernel_offsets_check(int offsets_dtype);
 
 #define RG_SET(OP, T, OFFT, VEC, FLAT, MASK)                                              \
   {(const void*)&rg::k_naive<OP, T, OFFT, VEC, FLAT, MASK>,                               \
+   rg::naive_held_kernel<OP, T, OFFT, VEC, FLAT, MASK>(),                                 \
    (const void*)&rg::k_worker<OP, T, OFFT, VEC, FLAT, MASK>,                              \
    rg::fused_kernel<OP, T, OFFT, VEC, FLAT, MASK, std::is_same<T, float>::value>(),              \
    rg::fused_kernel<OP, T, OFFT, VEC, FLAT, MASK, true>(),                                       \
@@ -92,7 +101,7 @@ const void* kernel_offsets_check(int offsets_dtype);
 #define RG_GEOMETRIES(OP, OFFT, MASK)                                                           \
   {{RG_SET(OP, float, OFFT, 1, false, MASK), RG_SET(OP, float, OFFT, 2, false, MASK),          \
     RG_SET(OP, float, OFFT, 4, false, MASK), RG_SET(OP, float, OFFT, 4, true, MASK),           \
-    {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, false, 0, 0}},                                      \
+    {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, false, 0, 0}},                                      \
    {RG_SET(OP, __bf16, OFFT, 1, false, MASK), RG_SET(OP, __bf16, OFFT, 2, false, MASK),        \
     RG_SET(OP, __bf16, OFFT, 4, false, MASK), RG_SET(OP, __bf16, OFFT, 8, false, MASK),        \
     RG_SET(OP, __bf16, OFFT, 8, true, MASK)}}

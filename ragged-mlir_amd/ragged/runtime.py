@@ -832,7 +832,7 @@ class CompiledProgram:
 
     def _kernel_name(self, role: str) -> str:
         phase = "online" if self.spec.op == "softmax" else self.spec.op
-        manifest_role = {"worker": f"worker_{phase}", "naive": phase, "fused": "fused_online",
+        manifest_role = {"worker": f"worker_{phase}", "naive": phase, "block": phase, "fused": "fused_online",
                          "deferred": "deferred_online"}.get(role, role)
         return self._names.get(manifest_role, f"ragged_0_{manifest_role}")
 

@@ -1,0 +1,40 @@
+"""Block-per-segment softmax that holds a segment in a workgroup's registers
+(csrc/held.hpp), against the oracle at its edges: segments of one row, of
+exactly the rows it holds, one more (streamed), the array's end inside a
+vector, and columns with -inf, NaN and only -inf; and the streaming kernel a
+call of longer mean segments takes."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from ragged import Compiler, ProgramSpec
+from ragged.workloads import offsets_from_lengths
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype,d", [("f32", 1), ("f32", 2), ("f32", 16), ("f32", 25), ("f32", 300), ("bf16", 1),
+                                     ("bf16", 4), ("bf16", 5), ("bf16", 64), ("bf16", 84)])
+def test_held_segments(artifact_cache, dtype, d):
+    from gpu_helpers import check, run_program
+    program = Compiler().compile(ProgramSpec("softmax", dtype, d, "i64", scale=1.25), artifact_cache)
+    size = 2 if dtype == "bf16" else 4
+    vec = program.metadata["d_vector"]
+    if program.metadata["mapping"] == "flat":
+        held = 8 * 256 * 16 // (d * size)
+    else:
+        lanes = 1
+        while lanes < -(-d // vec) and lanes < 256:
+            lanes *= 2
+        held = 16 * (256 // lanes)
+    rng = np.random.default_rng(d)
+    for lengths in ([1, 0, 2, held, 7], [held + 1, 3, held - 1, 0], [held] * 2 + [5] * 40, [6 * held, 2]):
+        offsets = offsets_from_lengths(np.array(lengths, dtype=np.int64), "i64")
+        values = rng.normal(size=(int(offsets[-1]), d)).astype(np.float32) * 4
+        values[rng.random(values.shape) < 0.01] = -np.inf
+        values[int(offsets[-2]):, 0] = -np.inf
+        values[0, d - 1] = np.nan
+        actual, report = run_program(program, values, offsets, dtype=dtype, op="softmax", select="naive")
+        assert report.selected == "naive" and len(report.kernel_names) == 1
+        check(actual, values, offsets, op="softmax", dtype=dtype, scale=1.25)
