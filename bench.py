@@ -250,28 +250,22 @@ def role_bytes(role: str, op: str, lengths: np.ndarray, d: int, element: int, t_
         if op == "softmax":
             return 2 * int(lengths.sum()) * d * element
         return (int(lengths.sum()) + len(lengths)) * d * element
-    if role == "naive":
+    if role == "split_partial":
+        # The tile kernel reads every row and writes every result (what
+        # crosses tiles is written by split_combine instead).
+        return (int(lengths.sum()) + len(lengths)) * d * element
+    if role == "split_combine":
+        return 0
+    if role in ("naive", "block"):       # block per segment, streaming or held in registers
         rows = lengths
     elif role == "wave":
         rows = lengths[lengths <= t_wave]
-    elif role == "block":
-        rows = lengths[(lengths > t_wave) & (lengths <= t_block)]
-    elif role in ("split_partial", "split_normalize", "split_combine"):
-        rows = lengths[lengths > t_block]
     else:
         return 0
     n_rows, segs = int(rows.sum()), int(len(rows))
     if op == "softmax":
-        if role == "split_partial":
-            return n_rows * d * element          # reads the rows once
-        if role == "split_normalize":
-            return n_rows * d * element          # writes the rows once (its re-read is not algorithmic)
-        if role == "split_combine":
-            return 0
         return 2 * n_rows * d * element
-    if role == "split_combine":
-        return segs * d * element                # writes the outputs
-    return n_rows * d * element + (0 if role == "split_partial" else segs * d * element)
+    return n_rows * d * element + segs * d * element
 
 
 def run_config(name: str, args, torch, cache, seed: int = 711) -> list[dict]:
