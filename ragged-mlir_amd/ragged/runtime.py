@@ -567,8 +567,8 @@ class CompiledProgram:
                 spec = self._native_spec()
                 module = _modules[key] = native.NativeModule(device, native.make_spec(
                     self.spec.op, self.spec.dtype, self.spec.offsets_dtype, self.spec.feature_dim,
-                    vectorize=self.spec.optimizations.vectorize, t_wave=int(spec.t_wave), t_block=t_block,
-                    part_rows=part_rows))
+                    scale=self.spec.scale, vectorize=self.spec.optimizations.vectorize, t_wave=int(spec.t_wave),
+                    t_block=t_block, part_rows=part_rows))
             return module
 
     def _plan(self, module: native.NativeModule, n: int, b: int, schedule: str) -> native.Plan:

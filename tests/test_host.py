@@ -300,3 +300,14 @@ def test_splits_segments_known_answers():
     assert splits_segments(4_194_304, 8192, 200_000, 1024)     # C5 lengths with max_len
     assert not splits_segments(4_194_304, 8192, None, 1024)    # ... and without: not provable
     assert not splits_segments(0, 0, None, 1024)
+
+
+def test_companion_modules_keep_the_scale(tmp_path, monkeypatch):
+    """The companion of a scaled sum with larger split parts applies the scale."""
+    from ragged import ArtifactCache, Compiler, ProgramSpec, runtime
+    program = Compiler().compile(ProgramSpec("sum", "f32", 128, "i64", scale=2.5), ArtifactCache(tmp_path))
+    made = []
+    monkeypatch.setattr(runtime.native, "NativeModule", lambda device, spec: made.append(spec) or object())
+    monkeypatch.setattr(runtime, "_modules", {})
+    program._parts_module(0, 4096, 2048)
+    assert made[0].scale == 2.5 and made[0].part_rows == 4096 and made[0].t_block == 2048
