@@ -549,7 +549,7 @@ static int plan_tiles(const rg_module* module, rg_plan* plan) {
     plan->buffer_bytes[index] = (uint64_t)bytes;
     end = offset + bytes;
   };
-  // (tiles * D * 8 is far below 2^63: a tile is at least 4 KiB of rows.)
+  // (tiles * D * 8 is far below 2^63: at most `wanted` tiles, or tiles of kTileMaxBytes.)
   buffer(RG_BUF_COUNTERS, (int64_t)kScratchCounterBytes);
   buffer(RG_BUF_ITEM_POS, tiles * 8);
   buffer(RG_BUF_PART_BEGIN, tiles * 8);

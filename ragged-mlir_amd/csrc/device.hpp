@@ -363,6 +363,13 @@ template <> struct State<OP_SUM> {
     c = __builtin_fabsf(t) < pos_inf() ? e : 0.f;
     s = t;
   }
+  // fold() where the sum is finite before and after; else s is not finite.
+  __device__ void fold_finite(float x) {
+    float y = x - c;
+    float t = s + y;
+    c = (t - s) - y;
+    s = t;
+  }
   __device__ float total() const { return s; }
   __device__ void merge(const State& o) { s = s + o.s; c = 0.f; }
   static constexpr float kIdentity = 0.f;

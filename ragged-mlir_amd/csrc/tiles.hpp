@@ -20,7 +20,7 @@
 //
 // Bound by memory: 539 MB f32 D=128 (4,096 segments of up to 512 rows) 107 ->
 // 91 us a call against the classified schedule, 5.9 TB/s, what a plain read
-// reaches; 1.07 GB bf16 D=128 long tail 238 -> 178 us (6.0 TB/s); 168 MB bf16
+// reaches; 1.07 GB bf16 D=128 long tail 235 -> 185 us (5.8 TB/s); 168 MB bf16
 // D=84 49 -> 40 us; 102 MB f32 D=2 29 -> 26 us; 100 MB f32 D=5 99 -> 49 us.
 // 128 KB: 12.7 -> 8.5 us of kernels, latency (launches, search, one batch).
 #pragma once
@@ -303,10 +303,7 @@ __global__ __launch_bounds__(kTileThreads) void k_tiles(Params p) {
     auto reduce = [&](int lanes) {
       xor_butterfly_range(lpr, lpr * lanes, [&](auto mask) {
 #pragma unroll
-        for (int v = 0; v < VEC; ++v) {
-          if constexpr (sizeof(T) == 4) merge_exact<OP>(st[v], shfl_xor_exact<decltype(mask)::value, OP>(st[v]));
-          else st[v].merge(shfl_xor<decltype(mask)::value, OP>(st[v]));
-        }
+        for (int v = 0; v < VEC; ++v) merge_exact<OP>(st[v], shfl_xor_exact<decltype(mask)::value, OP>(st[v]));
       });
     };
     auto put_partial = [&](int which) {
@@ -389,21 +386,26 @@ __global__ __launch_bounds__(kTileThreads) void k_tiles(Params p) {
             float x[K][VEC];
 #pragma unroll
             for (int u = 0; u < K; ++u) Elem<T>::template load<VEC>(at + (r - x0 + u * lanes) * d, x[u]);
+            bool folded = false;
             if constexpr (OP == OP_SUM && sizeof(T) == 2) {
-              // bf16 values: sums of a few 8-bit significands are exact or
-              // round far below the output's last bit, so one compensated
-              // add takes K rows.
+              // bf16 has twice the additions per byte: K rows are added
+              // without the check for an infinite sum after each, and once
+              // more with it where the result is not finite (the same bits).
+              State<OP> acc[VEC];
+              folded = true;
 #pragma unroll
-              for (int h = 1; h < K; h *= 2) {
+              for (int v = 0; v < VEC; ++v) {
+                acc[v] = st[v];
 #pragma unroll
-                for (int u = 0; u + h < K; u += 2 * h) {
-#pragma unroll
-                  for (int v = 0; v < VEC; ++v) x[u][v] = x[u][v] + x[u + h][v];
-                }
+                for (int u = 0; u < K; ++u) acc[v].fold_finite(x[u][v]);
+                folded = folded && __builtin_fabsf(acc[v].s) < pos_inf();
               }
+              if (folded) {
 #pragma unroll
-              for (int v = 0; v < VEC; ++v) st[v].fold(x[0][v]);
-            } else {
+                for (int v = 0; v < VEC; ++v) st[v] = acc[v];
+              }
+            }
+            if (!folded) {
 #pragma unroll
               for (int u = 0; u < K; ++u) {
 #pragma unroll

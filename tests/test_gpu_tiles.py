@@ -72,6 +72,24 @@ def test_tiles_element_access(artifact_cache, op, dtype, d):
     check(actual, values, offsets, op=op, dtype=dtype)
 
 
+@pytest.mark.parametrize("d", [4, 64, 84, 128])
+def test_tiles_bf16_sums_of_infinities(artifact_cache, d):
+    """Rows added several at a time and again one by one where a sum is not
+    finite: infinities of one sign, of both, and NaN, among finite columns."""
+    from gpu_helpers import check, run_program
+    program = Compiler().compile(ProgramSpec("sum", "bf16", d, "i64"), artifact_cache)
+    rng = np.random.default_rng(d)
+    lengths = np.concatenate([rng.integers(1, 200, 300), [60_000 // d]]).astype(np.int64)
+    offsets = offsets_from_lengths(lengths, "i64")
+    values = rng.normal(size=(int(offsets[-1]), d)).astype(np.float32)
+    values[rng.random(values.shape) < 0.004] = np.inf
+    values[:len(values) // 2][rng.random((len(values) // 2, d)) < 0.002] = -np.inf
+    values[rng.random(values.shape) < 0.001] = np.nan
+    actual, report = run_program(program, values, offsets, dtype="bf16", op="sum")
+    assert report.selection.get("tiles")
+    check(actual, values, offsets, op="sum", dtype="bf16")
+
+
 @pytest.mark.parametrize("op,dtype,d", [("sum", "f32", 2), ("sum", "bf16", 128), ("max", "f32", 100)])
 def test_tiles_repeat_bit_for_bit_and_share_a_workspace(artifact_cache, op, dtype, d):
     """The chains' order does not depend on scheduling, and a call on the
