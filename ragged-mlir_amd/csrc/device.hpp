@@ -476,21 +476,55 @@ __device__ __forceinline__ State<OP> shfl_xor(const State<OP>& a) {
   return r;
 }
 
+// The sum states of two lanes as one, with the rounding of their addition
+// kept (Knuth's two-sum): the true sum of a state is s - c.
+template <int OP>
+__device__ __forceinline__ void merge_exact(State<OP>& a, const State<OP>& b) {
+#pragma clang fp contract(off)
+  if constexpr (OP == OP_SUM) {
+    const float s = a.s + b.s;
+    const float bb = s - a.s;
+    const float e = (a.s - (s - bb)) + (b.s - bb);
+    a.c = (a.c + b.c) - e;
+    a.s = s;
+  } else {
+    a.merge(b);
+  }
+}
+template <int OP>
+__device__ __forceinline__ float exact_value(const State<OP>& a) {
+  if constexpr (OP == OP_SUM) return __builtin_isfinite(a.s) ? a.s - a.c : a.s;
+  else return a.m;
+}
+template <int MASK, int OP>
+__device__ __forceinline__ State<OP> shfl_xor_exact(const State<OP>& a) {
+  State<OP> r = shfl_xor<MASK, OP>(a);
+  if constexpr (OP == OP_SUM) r.c = xor_lane<MASK>(a.c);
+  return r;
+}
+
 // Combine lanes whose lane index agrees modulo `stride` (a power of two < 64):
 // afterwards every lane holds the combination over its residue class.
 template <int OP, int V>
 __device__ __forceinline__ void wave_reduce_stride(State<OP> (&st)[V], int stride) {
   xor_butterfly(stride, [&](auto mask) {
 #pragma unroll
-    for (int v = 0; v < V; ++v) st[v].merge(shfl_xor<decltype(mask)::value, OP>(st[v]));
+    for (int v = 0; v < V; ++v) merge_exact<OP>(st[v], shfl_xor_exact<decltype(mask)::value, OP>(st[v]));
   });
+  if constexpr (OP == OP_SUM) {
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+      st[v].s = exact_value<OP>(st[v]);
+      st[v].c = 0.f;
+    }
+  }
 }
 
 template <int OP> struct Slots { static constexpr int kCount = OP == OP_SOFTMAX ? 2 : 1; };
 
 template <int OP>
 __device__ __forceinline__ void st_write(float* slot, int stride, const State<OP>& a) {
-  if constexpr (OP == OP_SUM) { slot[0] = a.s; }
+  if constexpr (OP == OP_SUM) { slot[0] = exact_value<OP>(a); }
   else if constexpr (OP == OP_MAX) { slot[0] = a.m; }
   else { slot[0] = a.m; slot[stride] = a.s; }
 }

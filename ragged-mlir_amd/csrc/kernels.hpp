@@ -208,7 +208,7 @@ __device__ __forceinline__ void merge_components(State<OP> (&st)[VEC], int d) {
   for (int c = 1; c < VEC; ++c) {
 #pragma unroll
     for (int t = 0; t < c; ++t) {
-      if (c >= d && (c & (d - 1)) == t) st[t].merge(st[c]);
+      if (c >= d && (c & (d - 1)) == t) merge_exact<OP>(st[t], st[c]);
     }
   }
 }
@@ -249,7 +249,7 @@ __device__ __forceinline__ void block_reduce(State<OP> (&st)[VEC], int lpr, int 
       for (int v = 0; v < VEC; ++v) acc[v] = st_read<OP>(lds + (t * VEC + v) * S, 1);
       for (int ww = 1; ww < kWavesPerBlock; ++ww) {
 #pragma unroll
-        for (int v = 0; v < VEC; ++v) acc[v].merge(st_read<OP>(lds + ((ww * kWave + t) * VEC + v) * S, 1));
+        for (int v = 0; v < VEC; ++v) merge_exact<OP>(acc[v], st_read<OP>(lds + ((ww * kWave + t) * VEC + v) * S, 1));
       }
     } else {
       const int wpr = lpr / kWave;              // waves per row
@@ -258,7 +258,7 @@ __device__ __forceinline__ void block_reduce(State<OP> (&st)[VEC], int lpr, int 
       for (int v = 0; v < VEC; ++v) acc[v] = st_read<OP>(lds + ((w0 * kWave + l0) * VEC + v) * S, 1);
       for (int ww = w0 + wpr; ww < kWavesPerBlock; ww += wpr) {
 #pragma unroll
-        for (int v = 0; v < VEC; ++v) acc[v].merge(st_read<OP>(lds + ((ww * kWave + l0) * VEC + v) * S, 1));
+        for (int v = 0; v < VEC; ++v) merge_exact<OP>(acc[v], st_read<OP>(lds + ((ww * kWave + l0) * VEC + v) * S, 1));
       }
     }
   }

@@ -95,33 +95,6 @@ __device__ __forceinline__ void xor_butterfly_range(int lo, int hi, Step&& step)
   if (lo <= 32 && hi > 32) step(std::integral_constant<int, 32>{});
 }
 
-// The sum states of two lanes as one, with the rounding of their addition
-// kept (Knuth's two-sum): the true sum of a state is s - c.
-template <int OP>
-__device__ __forceinline__ void merge_exact(State<OP>& a, const State<OP>& b) {
-#pragma clang fp contract(off)
-  if constexpr (OP == OP_SUM) {
-    const float s = a.s + b.s;
-    const float bb = s - a.s;
-    const float e = (a.s - (s - bb)) + (b.s - bb);
-    a.c = (a.c + b.c) - e;
-    a.s = s;
-  } else {
-    a.merge(b);
-  }
-}
-template <int OP>
-__device__ __forceinline__ float exact_value(const State<OP>& a) {
-  if constexpr (OP == OP_SUM) return __builtin_isfinite(a.s) ? a.s - a.c : a.s;
-  else return a.m;
-}
-template <int MASK, int OP>
-__device__ __forceinline__ State<OP> shfl_xor_exact(const State<OP>& a) {
-  State<OP> r = shfl_xor<MASK, OP>(a);
-  if constexpr (OP == OP_SUM) r.c = xor_lane<MASK>(a.c);
-  return r;
-}
-
 // The chain of partials of tile w's head: out[s] = tail[first .. w-1], head[w]
 // in order, features f0 .. of `lanes` lanes per tile. Called by whole
 // workgroups of `threads` threads (it contains barriers).
