@@ -477,7 +477,10 @@ __device__ __forceinline__ State<OP> shfl_xor(const State<OP>& a) {
 }
 
 // The sum states of two lanes as one, with the rounding of their addition
-// kept (Knuth's two-sum): the true sum of a state is s - c.
+// kept (Knuth's two-sum): the true sum of a state is s - c. As in fold(), a
+// sum that is not finite has no correction (its e is inf - inf), so that a
+// later fold or merge of the state adds to s alone; nor has one whose two-sum
+// overflows on the way.
 template <int OP>
 __device__ __forceinline__ void merge_exact(State<OP>& a, const State<OP>& b) {
 #pragma clang fp contract(off)
@@ -485,7 +488,7 @@ __device__ __forceinline__ void merge_exact(State<OP>& a, const State<OP>& b) {
     const float s = a.s + b.s;
     const float bb = s - a.s;
     const float e = (a.s - (s - bb)) + (b.s - bb);
-    a.c = (a.c + b.c) - e;
+    a.c = __builtin_fabsf(e) < pos_inf() ? (a.c + b.c) - e : 0.f;
     a.s = s;
   } else {
     a.merge(b);

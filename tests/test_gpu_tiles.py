@@ -75,7 +75,8 @@ def test_tiles_element_access(artifact_cache, op, dtype, d):
 @pytest.mark.parametrize("d", [4, 64, 84, 128])
 def test_tiles_bf16_sums_of_infinities(artifact_cache, d):
     """Rows added several at a time and again one by one where a sum is not
-    finite: infinities of one sign, of both, and NaN, among finite columns."""
+    finite: short segments with infinities of one sign, of both, and NaN,
+    among finite columns."""
     from gpu_helpers import check, run_program
     program = Compiler().compile(ProgramSpec("sum", "bf16", d, "i64"), artifact_cache)
     rng = np.random.default_rng(d)
@@ -88,6 +89,45 @@ def test_tiles_bf16_sums_of_infinities(artifact_cache, d):
     actual, report = run_program(program, values, offsets, dtype="bf16", op="sum")
     assert report.selection.get("tiles")
     check(actual, values, offsets, op="sum", dtype="bf16")
+
+
+def extremes(n, d, rng):
+    """Finite values but for column 0 (one +inf) and, in rows of four or more, 1
+    (one -inf), 2 (both) and 3 (two finite values whose sum overflows); no NaN."""
+    values = rng.normal(size=(n, d)).astype(np.float32)
+    near, far = n // 5, n - n // 7
+    values[far, 0] = np.inf
+    if d > 3:
+        values[near, 1] = -np.inf
+        values[near, 2], values[far, 2] = np.inf, -np.inf
+        values[near, 3] = values[far, 3] = 3e38
+    return values
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("d,parts", [(1, 8), (1, 24), (1, 60), (1, 1000), (4, 24), (4, 60), (4, 900), (4, 1500), (64, 24),
+                                     (64, 60), (64, 200), (64, 900), (84, 100), (128, 600)])
+def test_tiles_infinite_sums_of_long_segments(artifact_cache, monkeypatch, dtype, d, parts):
+    """A sum that is infinite, or overflows, is infinite however many tiles
+    its segment crosses: chains a lane folds (up to 32 parts), a wave (64 per
+    lane group) and a workgroup, and those of a single workgroup of tiles."""
+    from gpu_helpers import run_program
+    monkeypatch.setattr(runtime, "SMALL_SEGMENTS", 0)
+    program = Compiler().compile(ProgramSpec("sum", dtype, d, "i64"), artifact_cache)
+    row = d * (2 if dtype == "bf16" else 4)
+    n = parts * (1 << 10 if parts <= 1000 else 4 << 10) // row
+    rng = np.random.default_rng(parts)
+    values = np.concatenate([rng.normal(size=(2, d)).astype(np.float32), extremes(n, d, rng),
+                             rng.normal(size=(3, d)).astype(np.float32)])
+    offsets = np.array([0, 2, n + 2, n + 5], dtype=np.int64)
+    for flip in (1, -1):
+        actual, report = run_program(program, values * np.float32(flip), offsets, dtype=dtype, op="sum")
+        assert report.selection.get("tiles")
+        assert np.isfinite(actual[[0, 2]]).all()
+        assert actual[1, 0] == flip * np.inf
+        if d > 3:
+            assert actual[1, 1] == -flip * np.inf and np.isnan(actual[1, 2]) and actual[1, 3] == flip * np.inf
+            assert np.isfinite(actual[1, 4:]).all()
 
 
 @pytest.mark.parametrize("op,dtype,d", [("sum", "f32", 2), ("sum", "bf16", 128), ("max", "f32", 100)])
