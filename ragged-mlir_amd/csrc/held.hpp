@@ -73,15 +73,15 @@ __device__ __forceinline__ bool held_softmax(const Params& p, int64_t start, int
   if constexpr (FLAT) fold_residues<true, VEC>(m, d);      // component c is feature c % D
   block_allreduce<true, VEC>(m, g.lpr, g.feat_lane, lds);
   ExpSum<T> acc[VEC];
-  ExpShift<T> ex[VEC];
+  float ref[VEC];
 #pragma unroll
-  for (int v = 0; v < VEC; ++v) ex[v] = ExpShift<T>(m[v] == neg_inf() ? 0.f : m[v]);
+  for (int v = 0; v < VEC; ++v) ref[v] = m[v] == neg_inf() ? 0.f : m[v];
 #pragma unroll
   for (int i = 0; i < K; ++i) {
     if (i * step >= count) break;
 #pragma unroll
     for (int v = 0; v < VEC; ++v) {
-      const float e = ex[v](value(i, v));
+      const float e = exp_out<T>(value(i, v) - ref[v]);
       acc[v].add(inside(i, v) ? e : 0.f);
       if constexpr (std::is_same<T, float>::value) w[i][v] = __float_as_uint(e);     // f32 keeps it for the output
     }
@@ -90,13 +90,9 @@ __device__ __forceinline__ bool held_softmax(const Params& p, int64_t start, int
   for (int v = 0; v < VEC; ++v) sum[v] = acc[v].s;
   if constexpr (FLAT) fold_residues<false, VEC>(sum, d);
   block_allreduce<false, VEC>(sum, g.lpr, g.feat_lane, lds);
-  Normalizer<T> norm[VEC];
   float inv[VEC];
 #pragma unroll
-  for (int v = 0; v < VEC; ++v) {
-    norm[v] = Normalizer<T>::of(m[v], sum[v]);
-    inv[v] = fast_exp(m[v] - m[v]) / sum[v];               // NaN for an all -inf column
-  }
+  for (int v = 0; v < VEC; ++v) inv[v] = fast_exp(m[v] - m[v]) / sum[v];     // 1 / sum, or NaN for an all -inf column
   T* out = static_cast<T*>(p.out);
 #pragma unroll
   for (int i = 0; i < K; ++i) {
@@ -106,7 +102,7 @@ __device__ __forceinline__ bool held_softmax(const Params& p, int64_t start, int
     float y[VEC];
 #pragma unroll
     for (int v = 0; v < VEC; ++v)
-      y[v] = std::is_same<T, float>::value ? __uint_as_float(w[i][v]) * inv[v] : norm[v](value(i, v));
+      y[v] = (std::is_same<T, float>::value ? __uint_as_float(w[i][v]) : exp_out<T>(value(i, v) - ref[v])) * inv[v];
     const int64_t e = FLAT ? j * VEC : j * d + g.feature;
     if (!FLAT || (e >= lo && e + VEC <= hi)) {
       Elem<T>::template store<VEC>(out + e, y);

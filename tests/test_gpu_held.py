@@ -38,3 +38,37 @@ def test_held_segments(artifact_cache, dtype, d):
         actual, report = run_program(program, values, offsets, dtype=dtype, op="softmax", select="naive")
         assert report.selected == "naive" and len(report.kernel_names) == 1
         check(actual, values, offsets, op="softmax", dtype=dtype, scale=1.25)
+
+
+def large_columns(offsets, d, rng):
+    """Logits whose columns are of very large magnitude, as padding and masks
+    make them: constant at -1e9, the lowest finite bf16 or 1e6, steps of an
+    ulp at -1e5 and 1e6, padding among ordinary values; and an ordinary one."""
+    lowest = -3.3895e38
+    kinds = [lambda k: np.full(k, -1e9), lambda k: np.full(k, lowest), lambda k: np.full(k, 1e6),
+             lambda k: -99840 - 512 * rng.integers(0, 2, k), lambda k: 999424 + 4096 * rng.integers(0, 2, k),
+             lambda k: np.where(rng.random(k) < 0.5, lowest, rng.normal(size=k)), lambda k: 2 * rng.normal(size=k)]
+    values = np.empty((int(offsets[-1]), d), dtype=np.float32)
+    for s, (start, end) in enumerate(zip(offsets[:-1], offsets[1:])):
+        for column in range(d):
+            values[start:end, column] = kinds[(s + column) % len(kinds)](int(end - start))
+    return values
+
+
+@pytest.mark.parametrize("select", ["naive"])
+@pytest.mark.parametrize("dtype,d", [("f32", 1), ("f32", 16), ("bf16", 1), ("bf16", 2), ("bf16", 25), ("bf16", 46),
+                                     ("bf16", 64), ("bf16", 84), ("bf16", 128)])
+def test_columns_of_large_magnitude(artifact_cache, dtype, d, select):
+    """exp(x - max) / sum depends on x - max alone, whatever the magnitude of
+    the column: short segments (held), and among them long ones (streamed;
+    chunks merged by all readers and by tree)."""
+    from gpu_helpers import check, run_program
+    program = Compiler().compile(ProgramSpec("softmax", dtype, d, "i64"), artifact_cache)
+    rng = np.random.default_rng(d)
+    for lengths in ([4, 30, 1, 0, 2, 50, 7] * 7, [4, 300, 1, 0, 40, 20_000 // min(d, 16), 7] * 2):
+        offsets = offsets_from_lengths(np.array(lengths, dtype=np.int64), "i64")
+        values = large_columns(offsets, d, rng)
+        actual, report = run_program(program, values, offsets, dtype=dtype, op="softmax", select=select,
+                                     max_len=max(lengths))
+        assert report.selected == select
+        check(actual, values, offsets, op="softmax", dtype=dtype)
