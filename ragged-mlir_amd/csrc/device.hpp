@@ -112,12 +112,13 @@ __device__ __forceinline__ float exp_out(float x) {
   if constexpr (std::is_same<T, float>::value) return exp_split(x);
   else return __expf(x);
 }
-// exp(x - ref) over rows of type T that share a column reference ref: bf16
-// rows as 2^(x log2(e) - ref log2(e)), one FMA into v_exp_f32 with
-// shift = -ref log2(e) computed once per column (the error of the rounded
-// shift, below 2^-24 |ref| log2(e) in the exponent, is far below a bf16
-// ulp); f32 rows through exp_split(x - ref). ±inf and NaN follow x - ref:
-// inf - inf and NaN give NaN, x - inf gives 0.
+// exp(x - ref) over rows of type T that share a column reference ref: f32
+// rows through exp_split, bf16 rows as 2^(x log2(e) - ref log2(e)), one FMA
+// into v_exp_f32 with shift = -ref log2(e) computed once per column. The
+// rounded shift is off by 2^-24 |ref| log2(e) in the exponent, 2^-16 (far
+// below a bf16 ulp) at kShiftReach; columns beyond it (wave_far) take
+// exp_out(x - ref). ±inf and NaN follow x - ref: inf - inf and NaN give NaN,
+// x - inf gives 0.
 template <class T>
 struct ExpShift {
   float ref = 0.f, shift = 0.f;
@@ -132,26 +133,49 @@ struct ExpShift {
 // The softmax output y = exp(x - M) / S of one column with statistics
 // (M, S), rounded once to T. bf16 outputs: y = 2^(x log2(e) - c) with
 // c = M log2(e) + log2(S), one FMA into v_exp_f32 per element (c is rounded
-// once per column; its error, below 2^-24 |c| in the exponent, is far below
-// a bf16 ulp), so no intermediate value can underflow before the output does.
-// f32 outputs: exp_split(x - M) * (1 / S), the reference's exp(x - m) / s
-// (ToGPU.cpp:712-733) with the division as a rounded reciprocal. Special
-// columns follow IEEE arithmetic: M = -inf (only -inf, S = 0), NaN M or S
-// give NaN everywhere; x = -inf in a finite column gives 0.
+// once per column, as ExpShift's shift is, with the same reach; beyond it
+// softmax_far), so no intermediate value can underflow before the output
+// does. f32 outputs: exp_split(x - M) * (1 / S), the reference's
+// exp(x - m) / s (ToGPU.cpp:712-733) with the division as a rounded
+// reciprocal. Special columns follow IEEE arithmetic: M = -inf (only -inf,
+// S = 0), NaN M or S give NaN everywhere; x = -inf in a finite column gives 0.
 template <class T>
 struct Normalizer {
   float a = 0.f, b = 0.f;   // bf16: a = -c; f32: a = M, b = 1 / S
   Normalizer() = default;
-  __device__ Normalizer(float a_, float b_) : a(a_), b(b_) {}
-  __device__ static Normalizer of(float m, float s) {
-    if constexpr (std::is_same<T, float>::value) return Normalizer(m, 1.0f / s);
-    else return Normalizer(-__builtin_fmaf(m, kLog2eHi, __builtin_amdgcn_logf(s)), 0.f);
+  // From (M, column_factor(S)).
+  __device__ Normalizer(float m, float factor) : a(m), b(factor) {
+    if constexpr (!std::is_same<T, float>::value) a = -__builtin_fmaf(m, kLog2eHi, factor);
   }
   __device__ float operator()(float x) const {
     if constexpr (std::is_same<T, float>::value) return exp_split(x - a) * b;
     else return __builtin_amdgcn_exp2f(__builtin_fmaf(x, kLog2eHi, a));
   }
 };
+// What a column's outputs need of its sum S: log2(S) (bf16), 1 / S (f32).
+template <class T>
+__device__ __forceinline__ float column_factor(float s) {
+  if constexpr (std::is_same<T, float>::value) return 1.0f / s;
+  else return __builtin_amdgcn_logf(s);
+}
+// The bf16 output of a column out of the shift's reach: the difference first.
+__device__ __forceinline__ float softmax_far(float x, float m, float log2_s) {
+  return __builtin_amdgcn_exp2f(__builtin_fmaf(x - m, kLog2eHi, -log2_s));
+}
+
+// Whether one of the wave's columns (VEC a lane) of maximum m is out of the
+// shift's reach, as padding at -1e9 or at the lowest finite value is: the wave
+// then subtracts first. (Subtracting always: 1.07 GB bf16 D=128 long tail 441 ->
+// 449 us a call.)
+constexpr float kShiftReach = 128.f;
+template <class T, int VEC>
+__device__ __forceinline__ bool wave_far(const float (&m)[VEC]) {
+  if constexpr (std::is_same<T, float>::value) return false;
+  bool far = false;
+#pragma unroll
+  for (int v = 0; v < VEC; ++v) far = far || __builtin_fabsf(m[v]) > kShiftReach;
+  return __ballot(far) != 0;
+}
 
 // Workgroup-wide OR of `x` for the kBlock-thread workgroups of every kernel
 // here: one ballot per wave, one LDS flag per wave, two barriers. HIP's

@@ -647,11 +647,20 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
         }
       }
     } else {
+      if (__builtin_expect(wave_far<T>(m), 0)) {
 #pragma unroll
-      for (int i = 0; i < RPT; ++i) {
-        if (!live(i)) continue;
+        for (int i = 0; i < RPT; ++i) {
+          if (!live(i)) continue;
 #pragma unroll
-        for (int v = 0; v < VEC; ++v) sum[v] += ex[v](Reg::get(data[i], v));
+          for (int v = 0; v < VEC; ++v) sum[v] += exp_out<T>(Reg::get(data[i], v) - ex[v].ref);
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < RPT; ++i) {
+          if (!live(i)) continue;
+#pragma unroll
+          for (int v = 0; v < VEC; ++v) sum[v] += ex[v](Reg::get(data[i], v));
+        }
       }
     }
 #pragma unroll
@@ -676,9 +685,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     bool defer = false;
     if (!chunk) {
       for (int f = t; f < d; f += kBlock) {
-        const Normalizer<T> n = Normalizer<T>::of(own_m[f], own_s[f]);
-        lds[f] = n.a;
-        lds_s[f] = n.b;
+        lds[f] = own_m[f];
+        lds_s[f] = column_factor<T>(own_s[f]);
       }
     } else {
       const int64_t idx = index_of(ticket);
@@ -699,11 +707,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
         defer = !ready;
         // Same thread wrote lds[f] / lds_s[f] in the fold: no barrier needed.
         if (ready) {
-          for (int f = t; f < d; f += kBlock) {
-            const Normalizer<T> n = Normalizer<T>::of(lds[f], lds_s[f]);
-            lds[f] = n.a;
-            lds_s[f] = n.b;
-          }
+          for (int f = t; f < d; f += kBlock) lds_s[f] = column_factor<T>(lds_s[f]);
         }
       }
       if (t == 0 && defer) {
@@ -721,20 +725,38 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
       //    dropped by the resource's range check.
       const Rsrc out = make_rsrc(static_cast<T*>(p.out) + start * d, chunk_elems * (int64_t)sizeof(T));
       asm volatile("" : "+v"(voff));
-      Normalizer<T> norm[VEC];
+      float col_m[VEC], col_s[VEC];
 #pragma unroll
-      for (int v = 0; v < VEC; ++v) norm[v] = g.active ? Normalizer<T>(lds[g.feature + v], lds_s[g.feature + v])
-                                                       : Normalizer<T>();
+      for (int v = 0; v < VEC; ++v) {
+        col_m[v] = g.active ? lds[g.feature + v] : 0.f;
+        col_s[v] = g.active ? lds_s[g.feature + v] : 0.f;
+      }
       __builtin_amdgcn_s_setprio(3);
+      if (__builtin_expect(wave_far<T>(col_m), 0)) {
 #pragma unroll
-      for (int i = 0; i < RPT; ++i) {
-        if (!live(i)) continue;
-        float y[VEC];
+        for (int i = 0; i < RPT; ++i) {
+          if (!live(i)) continue;
+          float y[VEC];
 #pragma unroll
-        for (int v = 0; v < VEC; ++v) y[v] = norm[v](Reg::get(data[i], v));
-        uint32_t w[In::kCount];
-        In::set(w, y);
-        buffer_store<In::kBytes>(out, voff + i * step_in, 0, w);
+          for (int v = 0; v < VEC; ++v) y[v] = softmax_far(Reg::get(data[i], v), col_m[v], col_s[v]);
+          uint32_t w[In::kCount];
+          In::set(w, y);
+          buffer_store<In::kBytes>(out, voff + i * step_in, 0, w);
+        }
+      } else {
+        Normalizer<T> norm[VEC];
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) norm[v] = Normalizer<T>(col_m[v], col_s[v]);
+#pragma unroll
+        for (int i = 0; i < RPT; ++i) {
+          if (!live(i)) continue;
+          float y[VEC];
+#pragma unroll
+          for (int v = 0; v < VEC; ++v) y[v] = norm[v](Reg::get(data[i], v));
+          uint32_t w[In::kCount];
+          In::set(w, y);
+          buffer_store<In::kBytes>(out, voff + i * step_in, 0, w);
+        }
       }
       __builtin_amdgcn_s_setprio(0);
       if (p.visits && t == 0 && it.c == 0) atomicAdd(p.visits + it.seg, 1);
@@ -805,26 +827,37 @@ __device__ __forceinline__ bool finish_deferred(const Params& p, int64_t idx, in
   const bool ok = poll_fold<std::is_same<T, float>::value>(st.base, st.count, p.d, ticks, lds_m, lds_s, stage);
   if (!ok && !must) return false;
   for (int f = t; f < p.d; f += kBlock) {
-    const float nan = __builtin_nanf("");
-    const Normalizer<T> n = ok ? Normalizer<T>::of(lds_m[f], lds_s[f]) : Normalizer<T>(nan, nan);
-    lds_m[f] = n.a;
-    lds_s[f] = n.b;
+    if (!ok) lds_m[f] = __builtin_nanf("");
+    lds_s[f] = column_factor<T>(lds_s[f]);
   }
   __syncthreads();
   const RowGeo g = row_geo<VEC>(p.d, kBlock, t, 0);
+  // The register path's choice: the same lanes hold the same columns.
+  float col_m[VEC], col_s[VEC];
+  bool far = false;
+  auto column_constants = [&] {
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) {
+      col_m[v] = g.active ? lds_m[g.feature + v] : 0.f;
+      col_s[v] = g.active ? lds_s[g.feature + v] : 0.f;
+    }
+    far = wave_far<T>(col_m);
+  };
+  auto output = [&](int v, float x) {
+    if (!std::is_same<T, float>::value && far) return softmax_far(x, col_m[v], col_s[v]);
+    return Normalizer<T>(col_m[v], col_s[v])(x);
+  };
   if constexpr (MASK) {
     // Masked logits: one row step at a time (holding the mask's words as
     // well would spill the register path's rows).
     if (g.active) {
-      Normalizer<T> norm[VEC];
-#pragma unroll
-      for (int v = 0; v < VEC; ++v) norm[v] = Normalizer<T>(lds_m[g.feature + v], lds_s[g.feature + v]);
+      column_constants();
       T* out = static_cast<T*>(p.out);
       for (int64_t r = it.start + g.row_lane; r < it.start + it.rows; r += g.rows_step) {
         float x[VEC];
         load_input<T, VEC, MASK>(p, r * p.d + g.feature, x);
 #pragma unroll
-        for (int v = 0; v < VEC; ++v) x[v] = norm[v](x[v]);
+        for (int v = 0; v < VEC; ++v) x[v] = output(v, x[v]);
         Elem<T>::template store<VEC>(out + r * p.d + g.feature, x);
       }
     }
@@ -863,17 +896,14 @@ __device__ __forceinline__ bool finish_deferred(const Params& p, int64_t idx, in
       Reg::set(data[i], x);
     }
   }
-  Normalizer<T> norm[VEC];
-#pragma unroll
-  for (int v = 0; v < VEC; ++v) norm[v] = g.active ? Normalizer<T>(lds_m[g.feature + v], lds_s[g.feature + v])
-                                                   : Normalizer<T>();
+  column_constants();
   const Rsrc out = make_rsrc(static_cast<T*>(p.out) + it.start * p.d, elems * (int64_t)sizeof(T));
 #pragma unroll
   for (int i = 0; i < RPT; ++i) {
     if (i != 0 && wave_row0 + i * rstep >= it.rows) continue;
     float y[VEC];
 #pragma unroll
-    for (int v = 0; v < VEC; ++v) y[v] = norm[v](Reg::get(data[i], v));
+    for (int v = 0; v < VEC; ++v) y[v] = output(v, Reg::get(data[i], v));
     uint32_t w[In::kCount];
     In::set(w, y);
     buffer_store<In::kBytes>(out, voff + i * step, 0, w);

@@ -55,7 +55,7 @@ def large_columns(offsets, d, rng):
     return values
 
 
-@pytest.mark.parametrize("select", ["naive"])
+@pytest.mark.parametrize("select", ["naive", "classified"])
 @pytest.mark.parametrize("dtype,d", [("f32", 1), ("f32", 16), ("bf16", 1), ("bf16", 2), ("bf16", 25), ("bf16", 46),
                                      ("bf16", 64), ("bf16", 84), ("bf16", 128)])
 def test_columns_of_large_magnitude(artifact_cache, dtype, d, select):
@@ -72,3 +72,41 @@ def test_columns_of_large_magnitude(artifact_cache, dtype, d, select):
                                      max_len=max(lengths))
         assert report.selected == select
         check(actual, values, offsets, op="softmax", dtype=dtype)
+
+
+@pytest.mark.parametrize("select", ["naive", "classified"])
+@pytest.mark.parametrize("dtype,d", [("f32", 16), ("bf16", 16), ("bf16", 46), ("bf16", 128)])
+def test_masked_columns(artifact_cache, dtype, d, select):
+    """An additive mask of -1e9 over a whole column of a segment, over part of
+    one, and over none."""
+    from gpu_helpers import check, run_program
+    program = Compiler().compile(ProgramSpec("softmax", dtype, d, "i64", scale=0.125, mask=True), artifact_cache)
+    rng = np.random.default_rng(d)
+    lengths = [4, 300, 1, 0, 40, 20_000 // d, 7] * 2
+    offsets = offsets_from_lengths(np.array(lengths, dtype=np.int64), "i64")
+    values = 16 * rng.normal(size=(int(offsets[-1]), d)).astype(np.float32)
+    mask = np.zeros_like(values)
+    for s, (start, end) in enumerate(zip(offsets[:-1], offsets[1:])):
+        mask[start:end, s % 3::3] = -1e9
+        mask[start:end, (s + 1) % 3::3] = np.where(rng.random((end - start, len(range((s + 1) % 3, d, 3)))) < 0.5, -1e9, 0)
+    actual, report = run_program(program, values, offsets, dtype=dtype, op="softmax", select=select, mask=mask,
+                                 max_len=max(lengths))
+    assert report.selected == select
+    check(actual, values, offsets, op="softmax", dtype=dtype, mask=mask, scale=0.125)
+
+
+@pytest.mark.parametrize("dtype,d", [("bf16", 46), ("bf16", 128), ("bf16", 1024)])
+def test_large_columns_of_deferred_chunks(artifact_cache, dtype, d):
+    """Chunks that stop waiting are re-read with the same bits."""
+    from gpu_helpers import run_program
+    program = Compiler().compile(ProgramSpec("softmax", dtype, d, "i64"), artifact_cache)
+    offsets = offsets_from_lengths(np.array([3, 60_000 // d, 0, 400_000 // d, 5], dtype=np.int64), "i64")
+    values = large_columns(offsets, d, np.random.default_rng(d))
+    waited, _ = run_program(program, values, offsets, dtype=dtype, op="softmax", select="classified")
+    module = program._module(0)
+    module.set_spin_limit(0)
+    try:
+        deferred, _ = run_program(program, values, offsets, dtype=dtype, op="softmax", select="classified")
+    finally:
+        module.set_spin_limit(-1)
+    assert np.array_equal(waited, deferred)
