@@ -540,18 +540,31 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     //    same; the merges run at the base priority (raising them too gave
     //    back most of the gain).
     uint32_t data[RPT][Reg::kCount];
-    if constexpr (!STORE_F32) {
+    if constexpr (!MASK && In::kCount == Reg::kCount) {
+      // The registers hold the values' own words; f32 is scaled in place, all
+      // rows behind one branch (f32 D=46, 500,000 rows: 87.6 -> 76.7 us a call
+      // against words loaded aside and multiplied by a scale of 1).
       __builtin_amdgcn_s_setprio(3);
 #pragma unroll
       for (int i = 0; i < RPT; ++i) buffer_load<In::kBytes>(in, voff + i * step_in, 0, data[i]);
       __builtin_amdgcn_s_setprio(0);
+      if (STORE_F32 && p.has_scale) {
+#pragma unroll
+        for (int i = 0; i < RPT; ++i) {
+#pragma unroll
+          for (int w = 0; w < Reg::kCount; ++w) data[i][w] = __float_as_uint(__uint_as_float(data[i][w]) * p.scale);
+        }
+      }
     } else {
       // The mask's words land in the rows' registers, the values' words (raw)
-      // in registers of their own, kRawRows rows at a time (32 registers):
-      // every load of a group issues before the first is used. (A row's loads
-      // waited for the row before: bf16 D=16, 1,000,003 rows, scale and mask,
-      // 84 -> 56 us a call.)
-      constexpr int kRawRows = 32 / In::kCount < RPT ? 32 / In::kCount : RPT;
+      // in registers of their own, kRawRows rows at a time: every load of a
+      // group issues before the first is used (a row's loads waited for the
+      // row before: bf16 D=16, 1,000,003 rows, scale and mask, 107 -> 58 us a
+      // call), and none of the next group's, which would take registers the
+      // rows need (bf16 D=46, 500,000 rows, masked: 21 registers spilled, 118
+      // -> 102 us).
+      constexpr int kRawMost = VEC == 1 ? RPT : In::kCount > 2 ? 32 / In::kCount : 16;
+      constexpr int kRawRows = kRawMost < RPT ? kRawMost : RPT;
       __builtin_amdgcn_s_setprio(3);
       if constexpr (MASK) {
         const Rsrc mk = make_rsrc(p.mask + start * d, chunk_elems * 4);
@@ -563,6 +576,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
         uint32_t raw[kRawRows][In::kCount];
 #pragma unroll
         for (int i = 0; i < kRawRows; ++i) buffer_load<In::kBytes>(in, voff + (i0 + i) * step_in, 0, raw[i]);
+        __builtin_amdgcn_s_setprio(0);
 #pragma unroll
         for (int i = 0; i < kRawRows; ++i) {
 #pragma clang fp contract(off)
@@ -577,8 +591,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
           }
           Reg::set(data[i0 + i], x);
         }
+        __builtin_amdgcn_sched_barrier(0);
       }
-      __builtin_amdgcn_s_setprio(0);
     }
     // Next ticket, while the loads are in flight. A workgroup that could
     // wait for its segment takes it early only once every chunk of the
