@@ -810,6 +810,9 @@ static int enqueue(const char* entry, const rg_module* module, const rg_plan* pl
     const bool aligned = ((reinterpret_cast<uintptr_t>(values) | (uintptr_t)row) & 15) == 0;
     p.tile_batch = (int32_t)((rg::kTileStage - (aligned ? 0 : 16)) / row);
     p.tile_single = plan->launches == 1 && plan->items_cap > 1 ? 1 : 0;
+    // Flat-mapped results ([B, D], D below an access) may lie at any element:
+    // the row kernel then stores them one by one.
+    p.out_elements = module->geometry.flat && (reinterpret_cast<uintptr_t>(out) & (uintptr_t)(row - 1)) != 0 ? 1 : 0;
     p.counters = static_cast<int64_t*>(buffer(RG_BUF_COUNTERS));
     p.item_pos = static_cast<int64_t*>(buffer(RG_BUF_ITEM_POS));
     p.part_begin = static_cast<int64_t*>(buffer(RG_BUF_PART_BEGIN));

@@ -58,7 +58,7 @@ def test_tiles_match_the_oracle(artifact_cache, monkeypatch, op, dtype, d):
 
 @pytest.mark.parametrize("op,dtype,d", [("sum", "f32", 1), ("max", "bf16", 5), ("sum", "bf16", 16)])
 def test_tiles_element_access(artifact_cache, op, dtype, d):
-    """One element per access (unaligned views), non-finite values."""
+    """One element per access, non-finite values."""
     from gpu_helpers import check, run_program
     program = Compiler().compile(ProgramSpec(op, dtype, d, "i64", optimizations=Optimizations(vectorize=False)),
                                  artifact_cache)
@@ -70,6 +70,33 @@ def test_tiles_element_access(artifact_cache, op, dtype, d):
     actual, report = run_program(program, values, offsets, dtype=dtype, op=op)
     assert report.selection.get("tiles")
     check(actual, values, offsets, op=op, dtype=dtype)
+
+
+@pytest.mark.parametrize("op", ["sum", "max"])
+@pytest.mark.parametrize("dtype,d,vectorize", [("f32", 2, True), ("bf16", 2, True), ("bf16", 4, True), ("f32", 2, False),
+                                               ("f32", 6, False), ("bf16", 1, False), ("bf16", 4, False), ("bf16", 60, False)])
+def test_tiles_on_views_at_any_element(artifact_cache, monkeypatch, op, dtype, d, vectorize):
+    """Results of a flat-mapped program at any element of a buffer (its values
+    are aligned), and values and results of one with element accesses."""
+    from gpu_helpers import check, torch_dtype
+    monkeypatch.setattr(runtime, "SMALL_SEGMENTS", 0)
+    program = Compiler().compile(ProgramSpec(op, dtype, d, "i64", optimizations=Optimizations(vectorize=vectorize)),
+                                 artifact_cache)
+    rng = np.random.default_rng(d)
+    for lengths in (rng.integers(0, 90, 900), [5, 0, 9000, 3], [3]):
+        offsets = offsets_from_lengths(np.array(lengths, dtype=np.int64), "i64")
+        n, b = int(offsets[-1]), len(offsets) - 1
+        values = rng.normal(size=(n, d)).astype(np.float32)
+        for shift in (1, 3):
+            x = torch.zeros(n * d + 16, dtype=torch_dtype(torch, dtype), device="cuda")
+            y = torch.full((b * d + 16,), -64.0, dtype=x.dtype, device="cuda")
+            first = 0 if vectorize else shift
+            x[first:first + n * d] = torch.from_numpy(values).reshape(-1).to("cuda")
+            out = y[shift:shift + b * d].view(b, d)
+            report = program.run(x[first:first + n * d].view(n, d), torch.from_numpy(offsets).to("cuda"), out)
+            assert report.selection.get("tiles")
+            check(out.float().cpu().numpy().astype(np.float64), values, offsets, op=op, dtype=dtype)
+            assert bool((y[:shift] == -64).all()) and bool((y[shift + b * d:] == -64).all())
 
 
 @pytest.mark.parametrize("d", [4, 64, 84, 128])
