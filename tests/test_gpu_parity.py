@@ -171,16 +171,29 @@ def test_scale_and_mask(artifact_cache, dtype):
             check(actual, values, offsets, op=op, dtype=dtype, scale=-1.5)
 
 
-def test_unvectorized_unaligned_views(artifact_cache):
+@pytest.mark.parametrize("op,dtype", [("sum", "f32"), ("max", "bf16"), ("softmax", "f32"), ("softmax", "bf16")])
+def test_unvectorized_unaligned_views(artifact_cache, op, dtype):
     """vectorize=False accepts views at any element offset."""
+    import torch
     d = 8
-    program = Compiler().compile(ProgramSpec("sum", "f32", d, "i64", optimizations=Optimizations(vectorize=False)),
+    program = Compiler().compile(ProgramSpec(op, dtype, d, "i64", optimizations=Optimizations(vectorize=False)),
                                  artifact_cache)
     lengths = make_lengths("uniform", 50, seed=1, total_elements=5000)
     offsets = offsets_from_lengths(lengths, "i64")
     values = np.random.default_rng(2).normal(size=(int(offsets[-1]), d)).astype(np.float32)
-    actual, _ = run_program(program, values, offsets, dtype="f32", op="sum", select="classified")
-    check(actual, values, offsets, op="sum", dtype="f32")
+    actual, _ = run_program(program, values, offsets, dtype=dtype, op=op, select="classified")
+    check(actual, values, offsets, op=op, dtype=dtype)
+    rows = len(values) if op == "softmax" else len(offsets) - 1
+    for shift in (1, 3):
+        tdtype = torch.bfloat16 if dtype == "bf16" else torch.float32
+        x = torch.zeros(values.size + 16, dtype=tdtype, device="cuda")
+        x[shift:shift + values.size] = torch.from_numpy(values).reshape(-1).to("cuda")
+        y = torch.full((rows * d + 16,), -64.0, dtype=tdtype, device="cuda")
+        for select in ("classified", "naive"):
+            out = y[shift:shift + rows * d].view(rows, d)
+            program.run(x[shift:shift + values.size].view(-1, d), torch.from_numpy(offsets).to("cuda"), out, select=select)
+            check(out.float().cpu().numpy().astype(np.float64), values, offsets, op=op, dtype=dtype)
+            assert bool((y[:shift] == -64).all()) and bool((y[shift + rows * d:] == -64).all())
 
 
 @pytest.mark.parametrize("op", OPS)
