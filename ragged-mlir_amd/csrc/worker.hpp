@@ -281,7 +281,7 @@ __device__ __forceinline__ void lane_segment(const Params& p, int64_t s, int64_t
     T* out = static_cast<T*>(p.out) + s * p.d;
 #pragma unroll
     for (int f = 0; f < VEC; ++f) {
-      if (f < p.d) Elem<T>::put(out + f, value_of<OP>(st[f]));
+      if (f < p.d) Elem<T>::put(out + f, exact_value<OP>(st[f]));
     }
   }
   if (p.visits) atomicAdd(p.visits + s, 1);
@@ -447,12 +447,12 @@ __device__ __forceinline__ void split_part(const Params& p, int64_t item, int ti
     st_write<OP>(lds + t, kBlock, acc);
     __syncthreads();
     if (pl == 0 && f < p.d) {
-      for (int q = 1; q < pl_count; ++q) acc.merge(st_read<OP>(lds + q * ft + fl, kBlock));
+      for (int q = 1; q < pl_count; ++q) merge_exact<OP>(acc, st_read<OP>(lds + q * ft + fl, kBlock));
       if constexpr (OP == OP_SOFTMAX) {
         publish(p.stats_max + k * p.d + f, acc.m);
         publish(p.stats_sum + k * p.d + f, acc.s);
       } else {
-        Elem<T>::put(static_cast<T*>(p.out) + s * p.d + f, value_of<OP>(acc));
+        Elem<T>::put(static_cast<T*>(p.out) + s * p.d + f, exact_value<OP>(acc));
       }
     }
     __syncthreads();
