@@ -51,8 +51,19 @@ enum rg_index { RG_I32 = 0, RG_I64 = 1 };
  * rows and segment ends, one wave each, whatever the lengths are; a second
  * launch adds what crosses tiles (none for one tile; up to 16 tiles one
  * workgroup does both). items_cap is then the number of tiles and part_rows
- * the positions of a tile. */
-enum rg_schedule { RG_CLASSIFIED = 0, RG_BLOCK_PER_SEGMENT = 1, RG_SHORT_SEGMENTS = 2, RG_TILES = 3 };
+ * the positions of a tile.
+ * RG_HELD_SEGMENTS (softmax without a mask): RG_BLOCK_PER_SEGMENT for a call
+ * whose every segment the caller expects to be at most rg_spec_held_rows rows:
+ * held in registers by a workgroup unless they are too short for that to pay.
+ * A longer segment only runs slower. RG_BLOCK_PER_SEGMENT itself holds
+ * segments where N rows would fit, or, in the flat mapping, the mean. */
+enum rg_schedule {
+  RG_CLASSIFIED = 0,
+  RG_BLOCK_PER_SEGMENT = 1,
+  RG_SHORT_SEGMENTS = 2,
+  RG_TILES = 3,
+  RG_HELD_SEGMENTS = 4
+};
 
 /* Kernel roles (a plan lists its launches in submission order). */
 enum rg_role {
@@ -195,6 +206,10 @@ int rg_spec_defaults(rg_spec* spec);
 /* 1 if `spec` (after defaults) runs softmax through the register-resident
  * worker (RG_ROLE_FUSED), 0 if not, <0 on a bad spec. Host only. */
 int rg_spec_uses_fused(const rg_spec* spec);
+
+/* Longest segment, in rows, that RG_HELD_SEGMENTS is for (0: `spec` has no
+ * such schedule), <0 on a bad spec. Host only. */
+int64_t rg_spec_held_rows(const rg_spec* spec);
 
 /* Create a kernel specialisation on a device; replaces
  * DriverModule(cubin, target) (Driver.h:23-27, Driver.cpp:178-195). Fails with

@@ -67,13 +67,6 @@ constexpr int64_t kTileWavesPerCu = 12;
 constexpr int64_t kMarkerBytes = 256;
 constexpr int64_t kTileMaxBytes = 1 << 30;  // 32-bit offsets inside a tile
 
-// Block-per-segment softmax: up to this mean segment the kernel that holds
-// segments in registers (16 rows of 16 bytes per thread, half of that flat).
-// Measured per call, streaming -> held: bf16 D=64 41 KB longest 13.8 -> 9.1 us, 12
-// KB 36.1 -> 23.8; f32 D=1 10 KB 12.0 -> 8.2; bf16 D=1 100 B 180 -> 82; but 488
-// KB (bf16 D=128) 157 -> 174: streaming wants more workgroups per CU.
-constexpr int64_t kHeldBytes = 64 << 10;
-
 int element_bytes(int dtype) { return dtype == RG_BF16 ? 2 : 4; }
 
 // Geometry of a specialisation: elements per access and mapping, plus the
@@ -126,6 +119,52 @@ int64_t feature_tiles(int d, int vec, bool flat, int g) {
 int64_t marker_rows(const rg_spec& spec, const Geometry& geo) {
   const int64_t row = (int64_t)spec.feature_dim * element_bytes(spec.dtype);
   return std::max<int64_t>(1, (geo.flat ? kMarkerBytes / 4 : kMarkerBytes) / row);
+}
+
+// Block-per-segment softmax, held (csrc/held.hpp) or streaming. A workgroup
+// holds held_capacity rows; the held kernel runs at half the streaming one's
+// waves per SIMD, so it pays where segments fit, and where a thread's rows are
+// wide and more than one. Measured over 2,200 call shapes (4 and 48 MiB, six
+// length distributions), held time over streaming:
+//   flat                 0.46-1.03 all fit, up to 1.04 else: by the mean;
+//   rows of 8- and 16-byte accesses, longest segment above the capacity: bf16
+//     D=64, 128 0.87-1.17, D=84 up to 1.14, f32 D=46 1.0-1.71, D=128 up to
+//     1.54: streaming;
+//   fitting: bf16 D=16, 64, 128 (up to 16 lanes a row) 0.59-1.0 (tiny segments
+//     of D=128 up to 1.08); f32 D=16-256 and bf16 D=84-256 0.74-1.0 from a mean of
+//     capacity / 16 (a row per thread) on, below it up to 1.59; rows of more
+//     than 32 lanes f32 D=256-1024 0.74-1.06 from capacity / 4 on, up to 1.76
+//     below; bf16 D=500, 1024 1.0-1.66: streaming;
+//   4-byte accesses (bf16 D=46, f32 D=5, 25): 0.83-1.0 up to capacity / 4, at the
+//     capacity up to 1.15; 2-byte (bf16 D=5, 25): 0.86-1.24, streaming.
+// Lanes per row of a workgroup.
+int64_t row_lanes(int d, const Geometry& geo) { return next_pow2_capped((d + geo.vec - 1) / geo.vec, rg::kBlock); }
+
+int64_t held_capacity(int d, const Geometry& geo) {
+  return geo.flat ? (int64_t)rg::kHeldRows<true> * rg::kBlock * geo.vec / d
+                  : rg::kHeldRows<false> * (rg::kBlock / row_lanes(d, geo));
+}
+
+// Longest segment the held kernel takes (0: none).
+int64_t held_rows(const rg_spec& spec, const Geometry& geo) {
+  if (spec.op != RG_OP_SOFTMAX || spec.has_mask) return 0;
+  const int64_t capacity = held_capacity(spec.feature_dim, geo);
+  if (geo.flat) return capacity - geo.vec / spec.feature_dim;      // (a segment may begin inside a vector)
+  const int access = geo.vec * element_bytes(spec.dtype);
+  if (spec.dtype == RG_BF16 && row_lanes(spec.feature_dim, geo) > 32) return 0;
+  return access >= 8 ? capacity : access == 4 ? capacity / 4 : 0;
+}
+
+// Whether a call of (n, b) rows and segments, the longest at most `longest`
+// rows, holds its segments.
+bool holds_segments(const rg_spec& spec, const Geometry& geo, int64_t n, int64_t b, int64_t longest) {
+  const int64_t rows = held_rows(spec, geo);
+  if (rows == 0 || n == 0) return false;
+  if (geo.flat) return (n - 1) / held_capacity(spec.feature_dim, geo) < b;
+  if (longest > rows) return false;
+  const int64_t lanes = row_lanes(spec.feature_dim, geo), capacity = held_capacity(spec.feature_dim, geo);
+  if (spec.dtype == RG_BF16 && lanes <= 16 && geo.vec >= 4) return true;
+  return n / std::max<int64_t>(1, capacity / (lanes > 32 ? 4 : 16)) >= b;
 }
 
 int combine_features_host(int d) { return next_pow2_capped(d, rg::kCombineFeatures); }
@@ -302,6 +341,14 @@ int rg_spec_uses_fused(const rg_spec* spec_in) {
   const int64_t capacity = fused_capacity(spec.dtype, spec.feature_dim, geo.vec, geo.flat,
                                           spec.has_mask != 0 || spec.scale != 1.0f);
   return capacity > 0 && spec.t_block <= capacity && spec.part_rows <= capacity ? 1 : 0;
+}
+
+int64_t rg_spec_held_rows(const rg_spec* spec_in) {
+  if (!spec_in) return fail(RG_E_INVALID, "rg_spec_held_rows: null spec");
+  rg_spec spec = *spec_in;
+  const int status = rg_spec_defaults(&spec);
+  if (status) return status;
+  return held_rows(spec, choose_geometry(spec.dtype, spec.feature_dim, spec.vectorize != 0));
 }
 
 int rg_module_create(int device, const rg_spec* spec_in, rg_module** out) {
@@ -569,12 +616,14 @@ int rg_plan_create(const rg_module* module, int64_t n, int64_t b, int schedule, 
   if (n < 0 || b < 0) return fail(RG_E_INVALID, "N and B must be nonnegative");
   if (b == 0 && n != 0) return fail(RG_E_INVALID, "B=0 requires N=0");
   if (schedule != RG_CLASSIFIED && schedule != RG_BLOCK_PER_SEGMENT && schedule != RG_SHORT_SEGMENTS &&
-      schedule != RG_TILES)
+      schedule != RG_TILES && schedule != RG_HELD_SEGMENTS)
     return fail(RG_E_INVALID, "unknown schedule");
   if (schedule == RG_SHORT_SEGMENTS && (module->spec.t_wave < 1 || module->spec.alone_rows < 1))
     return fail(RG_E_INVALID, "this specialisation has no short-segment schedule");
-  if (schedule == RG_BLOCK_PER_SEGMENT && module->spec.debug_visits)
+  if ((schedule == RG_BLOCK_PER_SEGMENT || schedule == RG_HELD_SEGMENTS) && module->spec.debug_visits)
     return fail(RG_E_INVALID, "debug visits require the classified schedule");
+  if (schedule == RG_HELD_SEGMENTS && held_rows(module->spec, module->geometry) == 0)
+    return fail(RG_E_INVALID, "this specialisation holds no segments");
   if (schedule == RG_TILES && (module->spec.op == RG_OP_SOFTMAX || module->spec.scale != 1.0f || module->spec.debug_visits))
     return fail(RG_E_INVALID, "the tile schedule takes sum and max without a scale or debug visits");
   if (schedule == RG_TILES && !module->roles[RG_ROLE_SPLIT_PARTIAL])
@@ -606,10 +655,9 @@ int rg_plan_create(const rg_module* module, int64_t n, int64_t b, int schedule, 
     plan->lds_bytes[i] = module->lds[role];
   };
   const int64_t tiles_block = feature_tiles(d, geo.vec, geo.flat, rg::kBlock);
-  if (schedule == RG_BLOCK_PER_SEGMENT) {
-    // A softmax whose mean segment a workgroup can hold holds them.
-    const bool held = module->roles[RG_ROLE_BLOCK] &&
-                      n <= b * ((geo.flat ? kHeldBytes / 2 : kHeldBytes) / (d * (int64_t)element_bytes(spec.dtype)));
+  if (schedule == RG_BLOCK_PER_SEGMENT || schedule == RG_HELD_SEGMENTS) {
+    // (Every segment of a call is at most N rows long.)
+    const bool held = holds_segments(spec, geo, n, b, schedule == RG_HELD_SEGMENTS ? held_rows(spec, geo) : n);
     add_launch(held ? RG_ROLE_BLOCK : RG_ROLE_NAIVE, b, tiles_block);
     return RG_OK;
   }

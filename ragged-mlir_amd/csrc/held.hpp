@@ -3,10 +3,14 @@
 //
 // Reading a segment twice (statistics, then the rows again) makes two chains
 // of rounds, each of a few loads, and two or more exponentials per element. A
-// segment of up to kHeldRows vectors per thread (64 KiB in 16-byte rows, 32 KiB
-// flat) is read once, every load in flight together; column max and column
+// segment of up to kHeldRows vectors (rows) per thread -- 64 KiB where rows take
+// 16-byte accesses and their lanes are a power of two, less elsewhere; 32 KiB
+// flat -- is read once, every load in flight together; column max and column
 // sum are exact passes over the registers, and the output is written from
-// them.
+// them. The registers cost half the waves per SIMD, so the plan takes this
+// kernel only where segments fit (holds_segments; bf16 D=64, 4 MiB in segments
+// of about 32 rows: 0.65 of the streaming kernel's time, of twice the
+// capacity: 1.06).
 #pragma once
 
 #include "fused.hpp"

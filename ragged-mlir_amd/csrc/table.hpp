@@ -67,7 +67,9 @@ constexpr const void* tiles_fold_kernel() {
 
 template <int OP, class T, class OFFT, int VEC, bool FLAT, bool MASK>
 constexpr const void* naive_held_kernel() {
-  if constexpr (OP == OP_SOFTMAX && !MASK) return (const void*)&k_naive<OP, T, OFFT, VEC, FLAT, false, true>;
+  // (Rows of 2-byte accesses always stream: held_rows.)
+  if constexpr (OP == OP_SOFTMAX && !MASK && VEC * (int)sizeof(T) > 2)
+    return (const void*)&k_naive<OP, T, OFFT, VEC, FLAT, false, true>;
   else return nullptr;
 }
 

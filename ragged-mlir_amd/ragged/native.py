@@ -21,7 +21,7 @@ ABI_VERSION = 3
 OPS = {"sum": 0, "max": 1, "softmax": 2}
 DTYPES = {"f32": 0, "bf16": 1}
 INDEX_DTYPES = {"i32": 0, "i64": 1}
-SCHEDULES = {"classified": 0, "naive": 1, "short": 2, "tiles": 3}
+SCHEDULES = {"classified": 0, "naive": 1, "short": 2, "tiles": 3, "held": 4}
 ROLES = ("init", "classify", "wave", "block", "split_partial", "split_combine", "split_normalize", "naive",
          "fused", "deferred", "worker")
 BUFFERS = ("class_counts", "segment_ids", "item_segments", "part_begin", "partials", "partial_sums",
@@ -81,6 +81,7 @@ def _declare(lib: ctypes.CDLL) -> ctypes.CDLL:
         "rg_device_query": (c_int, [c_int, ctypes.POINTER(DeviceProps)]),
         "rg_spec_defaults": (c_int, [ctypes.POINTER(Spec)]),
         "rg_spec_uses_fused": (c_int, [ctypes.POINTER(Spec)]),
+        "rg_spec_held_rows": (c_i64, [ctypes.POINTER(Spec)]),
         "rg_module_create": (c_int, [c_int, ctypes.POINTER(Spec), ctypes.POINTER(vp)]),
         "rg_module_destroy": (None, [vp]),
         "rg_module_resident": (c_int, [vp, c_int, ctypes.POINTER(c_i64)]),
@@ -182,6 +183,15 @@ def uses_fused(spec: Spec) -> bool:
     if status < 0:
         _check(status, "rg_spec_uses_fused")
     return status == 1
+
+
+def held_rows(spec: Spec) -> int:
+    """Longest segment (rows) the block-per-segment softmax of ``spec`` is
+    meant to hold in registers (0: none)."""
+    rows = library().rg_spec_held_rows(ctypes.byref(spec))
+    if rows < 0:
+        _check(int(rows), "rg_spec_held_rows")
+    return int(rows)
 
 
 def interrupt_static(launches: int) -> None:

@@ -245,6 +245,7 @@ class CompiledProgram:
                        and lanes <= 64 and options.warp_mapping and options.split_mapping)
         self._names = {kernel["role"]: kernel["name"] for kernel in self._metadata["kernels"]}
         self._alone: int | None = None
+        self._held: int | None = None
         self._wait_limit: dict[int, int] = {}   # device -> longest segment (rows) the register path holds
         self._facts: tuple | None = None    # what _tensor_facts compares with
         self._torch_dtypes: tuple | None = None    # (values dtype, offsets dtype) as torch dtypes
@@ -452,6 +453,8 @@ class CompiledProgram:
             if self._short_segments(max_len):
                 schedule = "short"
                 selection = {**selection, "short_segments": True}
+            elif self._holds(n, max_len):
+                schedule = "held"
         elif schedule != "tiles":
             return None
         if stream is None:
@@ -508,6 +511,16 @@ class CompiledProgram:
         if self._alone is None:
             self._alone = int(self._native_spec().alone_rows)
         return self._alone
+
+    def _holds(self, n: int, max_len: int | None) -> bool:
+        """Whether every segment of this block-per-segment softmax call is
+        known to be short enough to be held in registers. A max_len that is
+        too small only costs time."""
+        if self.spec.op != "softmax" or self._schedule != "naive":
+            return False
+        if self._held is None:
+            self._held = native.held_rows(self._native_spec())
+        return 0 < self._held and (n if max_len is None else min(n, max_len)) <= self._held
 
     def _streams(self, values, n: int, b: int, max_len: int | None) -> bool:
         """Whether run(select="auto") takes the streaming schedule for this
@@ -648,7 +661,7 @@ class CompiledProgram:
                                      else ("classified", {}))
             if chosen == "naive":
                 return self.naive._run(values, offsets, out, stream, mode, debug_buffers=debug_buffers, mask=mask,
-                                       selected="naive", selection=selection)
+                                       selected="naive", selection=selection, max_len=max_len)
         else:
             selection = {"forced": True} if self.naive is not None else {}
         return self._run(values, offsets, out, stream, mode, debug_buffers=debug_buffers, mask=mask,
@@ -761,7 +774,7 @@ class CompiledProgram:
                 schedule = "short"
                 selection = {**selection, "short_segments": True}
             elif forced is None:
-                schedule = self._schedule
+                schedule = "held" if self._holds(n, max_len) else self._schedule
             if forced == "stream":
                 module = self._stream_module(device)
             elif schedule == "classified" and self.spec.op != "softmax" and not self.spec.debug_visits:

@@ -311,3 +311,16 @@ def test_companion_modules_keep_the_scale(tmp_path, monkeypatch):
     monkeypatch.setattr(runtime, "_modules", {})
     program._parts_module(0, 4096, 2048)
     assert made[0].scale == 2.5 and made[0].part_rows == 4096 and made[0].t_block == 2048
+
+
+def test_held_rows_of_specialisations():
+    """Rows a workgroup holds (16 per thread, flat 8 vectors): all of them in
+    rows of 8- and 16-byte accesses, a quarter of 4-byte ones, none of 2-byte
+    ones, of bf16 rows of more than 32 lanes, with a mask, or of a reduction."""
+    for op, dtype, d, mask, rows in (
+            ("softmax", "bf16", 64, False, 512), ("softmax", "bf16", 128, False, 256), ("softmax", "bf16", 84, False, 128),
+            ("softmax", "bf16", 46, False, 32), ("softmax", "bf16", 25, False, 0), ("softmax", "bf16", 500, False, 0),
+            ("softmax", "bf16", 1024, False, 0), ("softmax", "f32", 128, False, 128), ("softmax", "f32", 1024, False, 16),
+            ("softmax", "f32", 25, False, 32), ("softmax", "f32", 1, False, 8188), ("softmax", "bf16", 4, False, 4094),
+            ("softmax", "f32", 128, True, 0), ("sum", "f32", 128, False, 0)):
+        assert native.held_rows(native.make_spec(op, dtype, "i64", d, mask=mask)) == rows, (op, dtype, d, mask)
