@@ -145,6 +145,50 @@ def small_reduce(n: int, b: int, max_len: int | None, row_bytes: int, access_byt
             and longest * row_bytes <= SMALL_LONGEST_PER_ACCESS * access_bytes)
 
 
+# Other sum / max calls take the tiles unless another schedule is known to be
+# faster. Measured on 2,500 random calls (64 KiB-512 MiB, every width and length
+# distribution of the comparison suites), µs per call on the device:
+# - max_len at most what a lane group reduces alone: the worker over the
+#   segments in order is 0.73 of the tiles' time (0.49-0.99 for nine in ten; f32
+#   D=1, 2.8 M rows in 200,000 segments 12 against 17).
+# - max_len longer: a workgroup per segment has no search, no partials and one
+#   launch, but costs a dispatch per segment and, for the longest, one
+#   workgroup's rate; the two estimates below pick the faster of both within
+#   1.6% on average (always tiles: 8.7%; f32 D=3, 45 MB in 7,623 segments 13.7
+#   against 17.8, bf16 D=46, 57 MB in 7,593 segments 15.5 against 19.9).
+# - max_len unknown: many short segments of narrow rows, whose wave would
+#   merge lanes for each, are the classified worker's (0.88 of the tiles' time,
+#   at best 0.45; beyond 16 lanes a row no gain, and 1.1-1.7 of it from 16 rows
+#   on average).
+CLASSIFIED_SEGMENTS = 5000
+CLASSIFIED_MEAN_ROWS = 16
+CLASSIFIED_LANES = 16
+
+
+class ReduceEstimate:
+    """Device µs of a sum / max call as equal tiles and as a workgroup per
+    segment: launches, bytes, segments (the tiles' by the lanes a segment's end
+    merges) and the longest segment, fitted to the measurements above so that
+    the faster is picked (each within 25-40% rms: far from the line between
+    them either is far off without harm)."""
+
+    def __init__(self, row_bytes: int, access_bytes: int, element_bytes: int, lanes: int, flat: bool):
+        narrow, packed = 16 / access_bytes, 4 / element_bytes
+        self._row_mb = row_bytes / 2**20
+        self._tile_segment = 0.0043e-3 * (1 << (lanes - 1).bit_length()) ** 1.18 * packed ** 1.2
+        self._block_mb = 0.177 * narrow ** 0.15 * packed ** 0.18
+        self._block_segment = 4.1e-3 if flat else 1.28e-3
+        self._block_longest = 32.7 * narrow ** 0.74
+
+    def tiles(self, n: int, b: int) -> float:
+        return 12.7 + 0.158 * n * self._row_mb + self._tile_segment * b
+
+    def blocks(self, n: int, b: int, longest: int) -> float:
+        # (Whichever bounds the call, and some of the others.)
+        return 1.3 + ((self._block_mb * n * self._row_mb) ** 1.7 + (self._block_segment * b) ** 1.7
+                      + (self._block_longest * longest * self._row_mb) ** 1.7) ** (1 / 1.7)
+
+
 def splits_segments(n: int, b: int, max_len: int | None, t_block: int) -> bool:
     """Whether a call of (n, b, max_len) provably holds a segment longer than
     the block class (``t_block`` rows): by max_len, or else by more rows than
@@ -240,9 +284,12 @@ class CompiledProgram:
         options = spec.optimizations
         self._row_bytes = spec.feature_dim * (2 if spec.dtype == "bf16" else 4)
         self._access_bytes = self._metadata["d_vector"] * (2 if spec.dtype == "bf16" else 4)
-        lanes = 1 if self._metadata["mapping"] == "flat" else -(-spec.feature_dim // self._metadata["d_vector"])
+        flat = self._metadata["mapping"] == "flat"
+        self._lanes = lanes = 1 if flat else -(-spec.feature_dim // self._metadata["d_vector"])
         self._tiles = (spec.op != "softmax" and self._selects and float(self._metadata["scale"]) == 1.0
                        and lanes <= 64 and options.warp_mapping and options.split_mapping)
+        self._estimate = ReduceEstimate(self._row_bytes, self._access_bytes, 2 if spec.dtype == "bf16" else 4, lanes,
+                                        flat)
         self._names = {kernel["role"]: kernel["name"] for kernel in self._metadata["kernels"]}
         self._alone: int | None = None
         self._held: int | None = None
@@ -262,9 +309,13 @@ class CompiledProgram:
         return self._metadata
 
     def choose(self, n: int, b: int, max_len: int | None, l2_mib: float | None = None) -> tuple[str, dict[str, Any]]:
-        """The schedule ``run(select="auto")`` uses for this input, and why."""
+        """The schedule ``run(select="auto")`` uses for this input, and why
+        (before it, ``run`` takes a program's shorter cuts: every segment
+        reduced alone, the streaming schedule of long softmax segments)."""
         if self.naive is None:
             return self._schedule, {}
+        if self._tiles:
+            return self._reduce_route(n, b, max_len)
         key = (n, b, max_len, l2_mib)
         choice = self._choices.get(key)
         if choice is None:
@@ -276,6 +327,24 @@ class CompiledProgram:
                                                                  fused=bool(self._metadata["fused"]),
                                                                  flat=self._metadata["mapping"] == "flat")
         return choice
+
+    def _reduce_route(self, n: int, b: int, max_len: int | None) -> tuple[str, dict[str, Any]]:
+        """Schedule of a sum / max call that may take the tiles: "naive", or
+        "classified" -- as tiles where the reasons say so, else binned or,
+        every segment being short, in order."""
+        if small_reduce(n, b, max_len, self._row_bytes, self._access_bytes):
+            return "naive", {"max_len": max_len, "reason": "small call, short segments"}
+        if self._short_segments(max_len):
+            return "classified", {"max_len": max_len, "reason": "every segment reduced alone"}
+        if max_len is not None:
+            tiles, blocks = self._estimate.tiles(n, b), self._estimate.blocks(n, b, min(n, max_len))
+            if blocks < tiles:
+                return "naive", {"max_len": max_len, "reason": "block per segment estimated faster than tiles",
+                                 "estimated_us": {"tiles": round(tiles, 2), "naive": round(blocks, 2)}}
+        elif (b >= CLASSIFIED_SEGMENTS and n < CLASSIFIED_MEAN_ROWS * b and self._lanes <= CLASSIFIED_LANES
+              and self._metadata["mapping"] != "flat"):
+            return "classified", {"max_len": None, "reason": "many short segments of narrow rows"}
+        return "classified", {"max_len": max_len, "tiles": True}
 
     def close(self) -> None:
         """Drop this program's plans and workspaces; the shared native module
@@ -437,6 +506,9 @@ class CompiledProgram:
         torch = _torch_module
         if torch is None:
             return None
+        short = schedule is None and self._short_segments(max_len)
+        if schedule is None and not short and self._schedule == "classified" and self.spec.op != "softmax":
+            return None        # the part size of its split segments: _run
         facts = self._tensor_facts(torch, values, offsets, out, mask)
         if facts is None:
             return None
@@ -447,10 +519,8 @@ class CompiledProgram:
                 or not _device_runs.get((device, self.spec.chip))):
             return None
         if schedule is None:
-            if self._schedule == "classified" and self.spec.op != "softmax":
-                return None
             schedule = self._schedule
-            if self._short_segments(max_len):
+            if short:
                 schedule = "short"
                 selection = {**selection, "short_segments": True}
             elif self._holds(n, max_len):
@@ -628,18 +698,15 @@ class CompiledProgram:
             if select == "naive":
                 chosen, selection = "naive", {"forced": True}
             elif self._tiles:
-                # Sum / max: one workgroup per segment for small calls, else
-                # equal tiles of the input, whatever the lengths.
+                # Sum / max: equal tiles of the input, or what is known to be
+                # faster for its size.
                 try:
-                    small = small_reduce(values.shape[0], offsets.shape[0] - 1, max_len, self._row_bytes,
-                                         self._access_bytes)
+                    chosen, selection = self._reduce_route(int(values.shape[0]), offsets.shape[0] - 1, max_len)
                 except (AttributeError, IndexError, TypeError):
-                    small = False       # not tensors: validation reports it
-                if not small:
+                    chosen, selection = "classified", {"max_len": max_len, "tiles": True}     # validation reports it
+                if selection.get("tiles"):
                     return self._run(values, offsets, out, stream, mode, debug_buffers=debug_buffers, mask=mask,
-                                     selected="classified", selection={"max_len": max_len, "tiles": True},
-                                     schedule="tiles")
-                chosen, selection = "naive", {"max_len": max_len, "reason": "small call, short segments"}
+                                     selected="classified", selection=selection, schedule="tiles")
             elif self._short_segments(max_len):
                 # One worker launch reduces every segment alone: cheaper than
                 # both modelled schedules, so the model is not consulted.

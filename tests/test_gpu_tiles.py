@@ -44,6 +44,7 @@ def test_tiles_match_the_oracle(artifact_cache, monkeypatch, op, dtype, d):
     program = Compiler().compile(ProgramSpec(op, dtype, d, offsets_dtype), artifact_cache)
     launches = set()
     monkeypatch.setattr(runtime, "SMALL_SEGMENTS", 0)      # small calls too
+    monkeypatch.setattr(runtime, "CLASSIFIED_LANES", 0)    # and many short segments
     for elements in (700, 40_000, 900_000):
         for kind in ("tiny", "middle", "spread", "one"):
             offsets = offsets_from_lengths(lengths_of(kind, d, elements), offsets_dtype)
@@ -175,9 +176,11 @@ def test_tiles_repeat_bit_for_bit_and_share_a_workspace(artifact_cache, op, dtyp
 
 
 @pytest.mark.parametrize("op,dtype,d", [("sum", "f32", 1), ("max", "bf16", 5)])
-def test_small_calls_run_block_per_segment(artifact_cache, op, dtype, d):
+def test_small_calls_run_block_per_segment(artifact_cache, monkeypatch, op, dtype, d):
     """A call that fits the small rule is one launch; one segment more, one
-    row more or an unknown longest segment beyond it is not."""
+    row more or an unknown longest segment beyond it is not (larger calls'
+    estimates aside)."""
+    monkeypatch.setattr(runtime.ReduceEstimate, "blocks", lambda *_: float("inf"))
     from gpu_helpers import check, run_program
     program = Compiler().compile(ProgramSpec(op, dtype, d, "i32"), artifact_cache)
     row = d * (2 if dtype == "bf16" else 4)
@@ -185,10 +188,35 @@ def test_small_calls_run_block_per_segment(artifact_cache, op, dtype, d):
     rng = np.random.default_rng(2)
     for lengths, max_len, small in (([most, 0, 3], most, True), ([most, 0, 3], None, False), ([most - 3, 0, 3], None, True),
                                     ([most + 1, 5], most + 1, False), ([2] * runtime.SMALL_SEGMENTS, 2, True),
-                                    ([2] * (runtime.SMALL_SEGMENTS + 1), 2, False)):
+                                    ([70] * (runtime.SMALL_SEGMENTS + 1), 70, False)):
         offsets = offsets_from_lengths(np.array(lengths, dtype=np.int64), "i32")
         values = rng.normal(size=(int(offsets[-1]), d)).astype(np.float32)
         actual, report = run_program(program, values, offsets, dtype=dtype, op=op, max_len=max_len)
         assert report.selected == ("naive" if small else "classified")
         assert bool(report.selection.get("tiles")) != small
         check(actual, values, offsets, op=op, dtype=dtype)
+
+
+@pytest.mark.parametrize("op,dtype,d,lengths,max_len,route", [
+    # every segment reduced alone by a lane group (a small call: block per segment)
+    ("sum", "f32", 16, [32] * 5000, 32, "alone"), ("max", "bf16", 128, [7, 0, 32] * 3000, 32, "alone"),
+    ("sum", "f32", 16, [32] * 4096, 32, "naive"), ("sum", "f32", 16, [33] * 12_000, 33, "tiles"),
+    # many segments of some hundred rows, and with one that one workgroup would take long for
+    ("max", "f32", 3, [500] * 7600, 500, "naive"), ("max", "f32", 3, [500] * 7600 + [40_000], 40_000, "tiles"),
+    ("max", "f32", 3, [500] * 7600, None, "tiles"), ("sum", "bf16", 46, [80] * 7600, 80, "naive"),
+    # many short segments of unknown length: narrow rows, wide rows, fewer, longer
+    ("sum", "f32", 16, [10] * 5000, None, "classified"), ("sum", "f32", 128, [10] * 5000, None, "tiles"),
+    ("sum", "f32", 16, [10] * 4999, None, "tiles"), ("sum", "f32", 16, [16] * 5000, None, "tiles"),
+    ("sum", "f32", 1, [10] * 5000, None, "tiles")])
+def test_routes_of_reductions(artifact_cache, op, dtype, d, lengths, max_len, route):
+    from gpu_helpers import check, run_program
+    program = Compiler().compile(ProgramSpec(op, dtype, d, "i64"), artifact_cache)
+    offsets = offsets_from_lengths(np.array(lengths, dtype=np.int64), "i64")
+    values = np.random.default_rng(d).normal(size=(int(offsets[-1]), d)).astype(np.float32)
+    chosen, why = program.choose(len(values), len(lengths), max_len)
+    actual, report = run_program(program, values, offsets, dtype=dtype, op=op, max_len=max_len)
+    assert report.selected == chosen == ("naive" if route == "naive" else "classified")
+    assert bool(report.selection.get("tiles")) == bool(why.get("tiles")) == (route == "tiles")
+    assert bool(report.selection.get("short_segments")) == (route == "alone")
+    assert report.kernel_names[0].endswith("split_partial") == (route == "tiles")
+    check(actual, values, offsets, op=op, dtype=dtype)
