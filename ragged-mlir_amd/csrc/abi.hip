@@ -245,6 +245,7 @@ struct rg_module {
   const rg::KernelSet* kernels;
   const void* roles[RG_ROLE_COUNT];
   hipFunction_t functions[RG_ROLE_COUNT];   // of `roles`: launched without the runtime's lookup by symbol
+  hipFunction_t tiles_by_element;           // flat mapping: the tiles of one element per lane (unaligned results)
   int64_t resident[RG_ROLE_COUNT];
   uint32_t lds[RG_ROLE_COUNT];
   int64_t cu_count;
@@ -395,6 +396,7 @@ int rg_module_create(int device, const rg_spec* spec_in, rg_module** out) {
   // RG_ROLE_SPLIT_NORMALIZE stays empty: k_worker normalises split parts.
   module->roles[RG_ROLE_NAIVE] = k.naive;
   module->roles[RG_ROLE_BLOCK] = k.naive_held;
+  const void* tiles_by_element = nullptr;
   if (spec.op != RG_OP_SOFTMAX && feature_tiles(spec.feature_dim, module->geometry.vec, module->geometry.flat, rg::kWave) == 1) {
     // A narrow feature dimension (flat mapping elsewhere) is a row of one
     // D-element lane here.
@@ -403,6 +405,11 @@ int rg_module_create(int device, const rg_spec* spec_in, rg_module** out) {
                                                      : *rg::kernels_max(spec.dtype, spec.offsets_dtype, row_geometry);
     module->roles[RG_ROLE_SPLIT_PARTIAL] = rows.tiles;
     module->roles[RG_ROLE_SPLIT_COMBINE] = rows.tiles_fold;
+    if (module->geometry.flat) {
+      const rg::KernelSet& elements = spec.op == RG_OP_SUM ? *rg::kernels_sum(spec.dtype, spec.offsets_dtype, 0)
+                                                           : *rg::kernels_max(spec.dtype, spec.offsets_dtype, 0);
+      tiles_by_element = elements.tiles;
+    }
   }
   module->cu_count = prop.multiProcessorCount;
   const bool f32_logits = spec.has_mask != 0 || spec.scale != 1.0f;
@@ -438,6 +445,7 @@ int rg_module_create(int device, const rg_spec* spec_in, rg_module** out) {
   // group's last arriver, the last workgroup's drain) normally succeeds at
   // once; it polls for at most 1 s.
   module->fold_ticks = module->clock_khz * 1000;
+  if (err == hipSuccess && tiles_by_element) err = hipGetFuncBySymbol(&module->tiles_by_element, tiles_by_element);
   for (int role = 0; role < RG_ROLE_COUNT && err == hipSuccess; ++role) {
     module->resident[role] = 0;
     module->lds[role] = 0;
@@ -848,6 +856,7 @@ static int enqueue(const char* entry, const rg_module* module, const rg_plan* pl
     p.trace = module->trace;
     p.trace_cap = module->trace_cap;
   }
+  bool by_element = false;
   if (plan->schedule == RG_TILES) {
     p.tile_count = plan->items_cap;
     p.tile_items = plan->part_rows;
@@ -859,8 +868,8 @@ static int enqueue(const char* entry, const rg_module* module, const rg_plan* pl
     p.tile_batch = (int32_t)((rg::kTileStage - (aligned ? 0 : 16)) / row);
     p.tile_single = plan->launches == 1 && plan->items_cap > 1 ? 1 : 0;
     // Flat-mapped results ([B, D], D below an access) may lie at any element:
-    // the row kernel then stores them one by one.
-    p.out_elements = module->geometry.flat && (reinterpret_cast<uintptr_t>(out) & (uintptr_t)(row - 1)) != 0 ? 1 : 0;
+    // the kernel of one element per lane then stores them.
+    by_element = module->geometry.flat && (reinterpret_cast<uintptr_t>(out) & (uintptr_t)(row - 1)) != 0;
     p.counters = static_cast<int64_t*>(buffer(RG_BUF_COUNTERS));
     p.item_pos = static_cast<int64_t*>(buffer(RG_BUF_ITEM_POS));
     p.part_begin = static_cast<int64_t*>(buffer(RG_BUF_PART_BEGIN));
@@ -887,7 +896,8 @@ static int enqueue(const char* entry, const rg_module* module, const rg_plan* pl
     for (int i = 0; i < plan->launches; ++i) profile.call_roles.push_back(plan->roles[i]);
   }
   for (int i = 0; i < plan->launches && err == hipSuccess; ++i) {
-    const hipFunction_t fn = module->functions[plan->roles[i]];
+    const hipFunction_t fn = by_element && plan->roles[i] == RG_ROLE_SPLIT_PARTIAL ? module->tiles_by_element
+                                                                                   : module->functions[plan->roles[i]];
     if (!fn) {
       err = hipErrorInvalidDeviceFunction;
       break;

@@ -269,7 +269,6 @@ struct Params {
   int32_t tile_batch;      // rows a wave stages at once
   int32_t tile_single;     // one workgroup holds every tile and folds what crosses them
   int64_t marker_rows;     // positions a segment's end takes on that axis
-  int32_t out_elements;    // tile schedule: out is stored by element (a flat-mapped specialisation takes any alignment)
 };
 
 // ---------------------------------------------------------------------------

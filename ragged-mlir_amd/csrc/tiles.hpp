@@ -413,13 +413,7 @@ __global__ __launch_bounds__(kTileThreads) void k_tiles(Params p) {
           float x[VEC];
 #pragma unroll
           for (int v = 0; v < VEC; ++v) x[v] = exact_value<OP>(st[v]);
-          T* dst = out + (s + i) * d + g.feature;
-          if (VEC > 1 && p.out_elements) {
-#pragma unroll
-            for (int v = 0; v < VEC; ++v) Elem<T>::put(dst + v, x[v]);
-          } else {
-            Elem<T>::template store<VEC>(dst, x);
-          }
+          Elem<T>::template store<VEC>(out + (s + i) * d + g.feature, x);
         }
         init_all<OP, VEC>(st);
         open = false;
