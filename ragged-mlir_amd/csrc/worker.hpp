@@ -447,12 +447,12 @@ __device__ __forceinline__ void split_part(const Params& p, int64_t item, int ti
     st_write<OP>(lds + t, kBlock, acc);
     __syncthreads();
     if (pl == 0 && f < p.d) {
-      for (int q = 1; q < pl_count; ++q) merge_exact<OP>(acc, st_read<OP>(lds + q * ft + fl, kBlock));
+      for (int q = 1; q < pl_count; ++q) acc.merge(st_read<OP>(lds + q * ft + fl, kBlock));
       if constexpr (OP == OP_SOFTMAX) {
         publish(p.stats_max + k * p.d + f, acc.m);
         publish(p.stats_sum + k * p.d + f, acc.s);
       } else {
-        Elem<T>::put(static_cast<T*>(p.out) + s * p.d + f, exact_value<OP>(acc));
+        Elem<T>::put(static_cast<T*>(p.out) + s * p.d + f, value_of<OP>(acc));
       }
     }
     __syncthreads();

@@ -173,18 +173,16 @@ def test_scale_and_mask(artifact_cache, dtype):
 
 @pytest.mark.parametrize("select", ["auto", "classified", "naive"])
 def test_sums_keep_what_a_merge_rounds_off(artifact_cache, select):
-    """1 and three times 2^-25 in different lanes' or parts' shares of a sum
-    (each below half an ulp of 1) give the rounding of the exact total: the
-    components of one lane, the parts of a split segment."""
+    """1 and three times 2^-25 (each below half an ulp of 1) in different
+    lanes' shares of a sum, or components of one lane's, give the rounding of
+    the exact total."""
     program = Compiler().compile(ProgramSpec("sum", "f32", 1, "i64"), artifact_cache)
-    part = 65_536                  # rows of a split part
-    lengths = np.array([4, 8, 4 * part, 4], dtype=np.int64)
-    offsets = offsets_from_lengths(lengths, "i64")
+    offsets = offsets_from_lengths(np.array([4, 8, 60_000, 4], dtype=np.int64), "i64")
     values = np.zeros((int(offsets[-1]), 1), dtype=np.float32)
-    for start, step in ((0, 1), (4, 1), (12, part), (12 + 4 * part, 1)):
+    for start, step in ((0, 1), (4, 1), (12, 4), (60_012, 1)):
         values[start, 0] = 1
         values[start + step:start + 3 * step + 1:step, 0] = 2.0**-25
-    actual, _ = run_program(program, values, offsets, dtype="f32", op="sum", select=select, max_len=4 * part)
+    actual, _ = run_program(program, values, offsets, dtype="f32", op="sum", select=select)
     assert np.array_equal(actual, np.full((4, 1), 1 + 2.0**-23))
 
 
