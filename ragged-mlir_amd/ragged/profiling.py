@@ -164,8 +164,11 @@ def kernel_resources(path: Path) -> dict[str, dict[str, float]]:
 
 
 # Kernel-name patterns of the library's launch roles (bench.py --details keys).
+# (k_naive's seventh argument: holds segments in registers.)
 ROLE_PATTERNS = {"init": r"k_init\b", "classify": r"k_classify", "worker": r"k_worker",
-                 "fused": r"k_softmax_fused", "deferred": r"k_softmax_deferred", "naive": r"k_naive"}
+                 "fused": r"k_softmax_fused", "deferred": r"k_softmax_deferred",
+                 "naive": r"k_naive(?!<(?:[^,]*,){6} true>)", "block": r"k_naive<(?:[^,]*,){6} true>",
+                 "split_partial": r"k_tiles<", "split_combine": r"k_tiles_fold"}
 # rocprofv3 reports vgpr_count as (descriptor granules) x 4; gfx950 wave64
 # allocates VGPRs in granules of 8 (compiler remarks: 44 -> 24, 128 -> 64).
 VGPR_DECODE = 2

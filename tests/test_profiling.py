@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import json
 from pathlib import Path
+import re
 import sqlite3
 
 import pytest
@@ -30,6 +31,20 @@ def sql(query, *args):
 def test_short_names():
     assert profiling.short_name("void rg::k_worker<0, float, long, 4, true, false>(rg::Params)") == WORKER
     assert profiling.short_name("__amd_rocclr_copyBuffer") == "__amd_rocclr_copyBuffer"
+
+
+def test_every_launched_role_has_its_kernels():
+    """Each role's pattern takes its own kernels and no other role's."""
+    names = {"classify": ["k_classify<long>"], "worker": [WORKER], "fused": ["k_softmax_fused<bool _Accum, long, 8, 16, false, false>"],
+             "naive": ["k_naive<2, bool _Accum, long, 8, false, false, false>", "k_naive<2, float, int, 1, false, true, false>",
+                       "k_naive<0, float, long, 4, true, false>"],
+             "block": ["k_naive<2, bool _Accum, long, 8, false, false, true>", "k_naive<2, float, long, 4, true, false, true>"],
+             "split_partial": ["k_tiles<0, float, long, 4>", "k_tiles<1, bool _Accum, int, 4>"],
+             "split_combine": ["k_tiles_fold<1, float>"]}
+    for role, own in names.items():
+        for other, kernels in names.items():
+            for kernel in kernels:
+                assert bool(re.search(profiling.ROLE_PATTERNS[role], kernel)) == (role == other), (role, kernel)
 
 
 def test_kernel_stats_from_the_trace():
