@@ -146,16 +146,18 @@ def small_reduce(n: int, b: int, max_len: int | None, row_bytes: int, access_byt
 
 
 # Other sum / max calls take the tiles unless another schedule is known to be
-# faster. Measured on 2,500 random calls (64 KiB-512 MiB, every width and length
-# distribution of the comparison suites), µs per call on the device:
+# faster. Measured on 3,000 random calls (64 KiB-512 MiB, every width and length
+# distribution of the comparison suites, three inputs in turn), µs per call on
+# the device:
 # - max_len at most what a lane group reduces alone: the worker over the
-#   segments in order is 0.73 of the tiles' time (0.49-0.99 for nine in ten; f32
-#   D=1, 2.8 M rows in 200,000 segments 12 against 17).
+#   segments in order is 0.73 of the tiles' time (0.49-0.99 for nine in ten; bf16
+#   D=32, 40 MB in 39,419 segments 13 against 40).
 # - max_len longer: a workgroup per segment has no search, no partials and one
 #   launch, but costs a dispatch per segment and, for the longest, one
 #   workgroup's rate; the two estimates below pick the faster of both within
-#   1.6% on average (always tiles: 8.7%; f32 D=3, 45 MB in 7,623 segments 13.7
-#   against 17.8, bf16 D=46, 57 MB in 7,593 segments 15.5 against 19.9).
+#   1.1% on average over 2,000 other calls (always tiles: 7%; f32 D=3, 45 MB in
+#   7,623 segments 13.7 against 17.8, bf16 D=46, 57 MB in 7,593 segments 15.5
+#   against 19.9).
 # - max_len unknown: many short segments of narrow rows, whose wave would
 #   merge lanes for each, are the classified worker's (0.88 of the tiles' time,
 #   at best 0.45; beyond 16 lanes a row no gain, and 1.1-1.7 of it from 16 rows
@@ -175,18 +177,21 @@ class ReduceEstimate:
     def __init__(self, row_bytes: int, access_bytes: int, element_bytes: int, lanes: int, flat: bool):
         narrow, packed = 16 / access_bytes, 4 / element_bytes
         self._row_mb = row_bytes / 2**20
-        self._tile_segment = 0.0043e-3 * (1 << (lanes - 1).bit_length()) ** 1.18 * packed ** 1.2
-        self._block_mb = 0.177 * narrow ** 0.15 * packed ** 0.18
-        self._block_segment = 4.1e-3 if flat else 1.28e-3
-        self._block_longest = 32.7 * narrow ** 0.74
+        self._tile_segment = 0.0027e-3 * (1 << (lanes - 1).bit_length()) ** 1.31 * packed ** 1.18
+        self._block_mb = 0.179 * narrow ** 0.19 * packed ** 0.07
+        self._block_segment = 4.2e-3 if flat else 1.29e-3
+        self._block_longest = 35.0 * narrow ** 0.71
 
     def tiles(self, n: int, b: int) -> float:
-        return 12.7 + 0.158 * n * self._row_mb + self._tile_segment * b
+        return 12.6 + 0.163 * n * self._row_mb + self._tile_segment * b
 
     def blocks(self, n: int, b: int, longest: int) -> float:
-        # (Whichever bounds the call, and some of the others.)
-        return 1.3 + ((self._block_mb * n * self._row_mb) ** 1.7 + (self._block_segment * b) ** 1.7
-                      + (self._block_longest * longest * self._row_mb) ** 1.7) ** (1 / 1.7)
+        # Whichever bounds the call, and some of the others. (Beyond about 80
+        # MiB the inputs of successive calls leave the Infinity Cache, which the
+        # tiles' loads do not rely on.)
+        mb = n * self._row_mb
+        return 1.0 + ((self._block_mb * (mb + 0.46 * max(mb - 80.0, 0.0))) ** 1.38 + (self._block_segment * b) ** 1.38
+                      + (self._block_longest * longest * self._row_mb) ** 1.38) ** (1 / 1.38)
 
 
 def splits_segments(n: int, b: int, max_len: int | None, t_block: int) -> bool:
@@ -750,6 +755,9 @@ class CompiledProgram:
         fields.update(template)
         if not plan_names:
             fields["classes"] = ()
+        if selection and "tiles" in selection:
+            # No segment is binned by its length.
+            fields["classes"], fields["thresholds"] = ("tiles",) if plan_names else (), ()
         if selection and "t_block" in selection:
             # A companion module's block threshold (big_block_rows).
             thresholds = template["thresholds"]

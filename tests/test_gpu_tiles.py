@@ -219,4 +219,5 @@ def test_routes_of_reductions(artifact_cache, op, dtype, d, lengths, max_len, ro
     assert bool(report.selection.get("tiles")) == bool(why.get("tiles")) == (route == "tiles")
     assert bool(report.selection.get("short_segments")) == (route == "alone")
     assert report.kernel_names[0].endswith("split_partial") == (route == "tiles")
+    assert (report.classes == ("tiles",)) == (route == "tiles") and (route != "tiles" or report.thresholds == ())
     check(actual, values, offsets, op=op, dtype=dtype)
