@@ -297,7 +297,8 @@ class CompiledProgram:
                                         flat)
         self._names = {kernel["role"]: kernel["name"] for kernel in self._metadata["kernels"]}
         self._alone: int | None = None
-        self._held: int | None = None
+        self._short_limit: int | None = None    # longest segment of the short-segment schedule (-1: none)
+        self._held: int | None = None           # longest segment held by a block-per-segment softmax (-1: none)
         self._wait_limit: dict[int, int] = {}   # device -> longest segment (rows) the register path holds
         self._facts: tuple | None = None    # what _tensor_facts compares with
         self._torch_dtypes: tuple | None = None    # (values dtype, offsets dtype) as torch dtypes
@@ -591,11 +592,11 @@ class CompiledProgram:
         """Whether every segment of this block-per-segment softmax call is
         known to be short enough to be held in registers. A max_len that is
         too small only costs time."""
-        if self.spec.op != "softmax" or self._schedule != "naive":
-            return False
-        if self._held is None:
-            self._held = native.held_rows(self._native_spec())
-        return 0 < self._held and (n if max_len is None else min(n, max_len)) <= self._held
+        held = self._held
+        if held is None:
+            rows = native.held_rows(self._native_spec()) if self._schedule == "naive" else 0
+            held = self._held = rows if rows > 0 else -1
+        return held > 0 and (n if max_len is None or max_len > n else max_len) <= held
 
     def _streams(self, values, n: int, b: int, max_len: int | None) -> bool:
         """Whether run(select="auto") takes the streaming schedule for this
@@ -706,7 +707,7 @@ class CompiledProgram:
                 # Sum / max: equal tiles of the input, or what is known to be
                 # faster for its size.
                 try:
-                    chosen, selection = self._reduce_route(int(values.shape[0]), offsets.shape[0] - 1, max_len)
+                    chosen, selection = self._reduce_route(values.shape[0], offsets.shape[0] - 1, max_len)
                 except (AttributeError, IndexError, TypeError):
                     chosen, selection = "classified", {"max_len": max_len, "tiles": True}     # validation reports it
                 if selection.get("tiles"):
@@ -755,13 +756,14 @@ class CompiledProgram:
         fields.update(template)
         if not plan_names:
             fields["classes"] = ()
-        if selection and "tiles" in selection:
-            # No segment is binned by its length.
-            fields["classes"], fields["thresholds"] = ("tiles",) if plan_names else (), ()
-        if selection and "t_block" in selection:
-            # A companion module's block threshold (big_block_rows).
-            thresholds = template["thresholds"]
-            fields["thresholds"] = (thresholds[0], selection["t_block"]) + thresholds[2:]
+        if selection:
+            if "tiles" in selection:
+                # No segment is binned by its length.
+                fields["classes"], fields["thresholds"] = ("tiles",) if plan_names else (), ()
+            elif "t_block" in selection:
+                # A companion module's block threshold (big_block_rows).
+                thresholds = template["thresholds"]
+                fields["thresholds"] = (thresholds[0], selection["t_block"]) + thresholds[2:]
         fields["grids"] = tuple(grids)
         fields["workspace_bytes"] = workspace + validation_bytes
         fields["mode"] = mode
@@ -778,10 +780,15 @@ class CompiledProgram:
         every segment alone: then one worker launch takes the segments in
         order (no classify, no workspace). A max_len that is too small only
         costs time."""
-        thresholds = self._metadata["thresholds"]
-        return (self._schedule == "classified" and max_len is not None
-                and not self.spec.debug_visits and bool(thresholds) and 0 < thresholds[0]
-                and 0 < self._alone_rows() and max_len <= self._alone_rows())
+        if max_len is None:
+            return False
+        limit = self._short_limit
+        if limit is None:
+            thresholds = self._metadata["thresholds"]
+            able = (self._schedule == "classified" and not self.spec.debug_visits and bool(thresholds)
+                    and 0 < thresholds[0] and 0 < self._alone_rows())
+            limit = self._short_limit = self._alone_rows() if able else -1
+        return max_len <= limit
 
     def _run(self, values, offsets, out, stream, mode, *, debug_buffers, mask, selected, selection,
              max_len: int | None = None, schedule: str | None = None) -> ExecutionReport:
