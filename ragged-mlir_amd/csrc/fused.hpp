@@ -542,12 +542,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     uint32_t data[RPT][Reg::kCount];
     if constexpr (!MASK && In::kCount == Reg::kCount) {
       // The registers hold the values' own words; f32 is scaled in place, all
-      // rows behind one branch (f32 D=46, 500,000 rows: 87.6 -> 76.7 us a call
-      // against words loaded aside and multiplied by a scale of 1).
-      __builtin_amdgcn_s_setprio(3);
+      // rows behind one branch (f32 D=46, 500,000 rows: 87.6 -> 75.9 us a call
+      // against words loaded aside and multiplied by a scale of 1). f32 loads
+      // issue at the base priority (raised: f32 D=128, 262,144 rows 72.1 -> 73.3 us).
+      if (!STORE_F32) __builtin_amdgcn_s_setprio(3);
 #pragma unroll
       for (int i = 0; i < RPT; ++i) buffer_load<In::kBytes>(in, voff + i * step_in, 0, data[i]);
-      __builtin_amdgcn_s_setprio(0);
+      if (!STORE_F32) __builtin_amdgcn_s_setprio(0);
       if (STORE_F32 && p.has_scale) {
 #pragma unroll
         for (int i = 0; i < RPT; ++i) {
