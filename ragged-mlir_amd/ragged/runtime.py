@@ -321,6 +321,8 @@ class CompiledProgram:
         if self.naive is None:
             return self._schedule, {}
         if self._tiles:
+            if max_len is not None and l2_mib is not None and not (isinstance(l2_mib, (int, float)) and l2_mib > 0):
+                raise ValueError("l2_mib must be a positive capacity in MiB")
             return self._reduce_route(n, b, max_len)
         key = (n, b, max_len, l2_mib)
         choice = self._choices.get(key)
