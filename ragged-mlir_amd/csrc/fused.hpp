@@ -847,32 +847,32 @@ __device__ __forceinline__ bool finish_deferred(const Params& p, int64_t idx, in
   }
   __syncthreads();
   const RowGeo g = row_geo<VEC>(p.d, kBlock, t, 0);
-  // The register path's choice: the same lanes hold the same columns.
-  float col_m[VEC], col_s[VEC];
-  bool far = false;
-  auto column_constants = [&] {
+  // The register path's choice of arithmetic: the same lanes hold the same
+  // columns. (Their constants are read from LDS row by row: held, they would
+  // not fit beside the rows of a whole item, and a kernel with any scratch
+  // takes about 1.8 us longer to launch.)
+  const int feature = g.active ? g.feature : 0;
+  auto is_far = [&] {
+    float col_m[VEC];
 #pragma unroll
-    for (int v = 0; v < VEC; ++v) {
-      col_m[v] = g.active ? lds_m[g.feature + v] : 0.f;
-      col_s[v] = g.active ? lds_s[g.feature + v] : 0.f;
-    }
-    far = wave_far<T>(col_m);
+    for (int v = 0; v < VEC; ++v) col_m[v] = g.active ? lds_m[feature + v] : 0.f;
+    return wave_far<T>(col_m);
   };
-  auto output = [&](int v, float x) {
-    if (!std::is_same<T, float>::value && far) return softmax_far(x, col_m[v], col_s[v]);
-    return Normalizer<T>(col_m[v], col_s[v])(x);
+  auto output = [&](bool far, int f, int v, float x) {
+    if (!std::is_same<T, float>::value && far) return softmax_far(x, lds_m[f + v], lds_s[f + v]);
+    return Normalizer<T>(lds_m[f + v], lds_s[f + v])(x);
   };
   if constexpr (MASK) {
     // Masked logits: one row step at a time (holding the mask's words as
     // well would spill the register path's rows).
     if (g.active) {
-      column_constants();
+      const bool far = is_far();
       T* out = static_cast<T*>(p.out);
       for (int64_t r = it.start + g.row_lane; r < it.start + it.rows; r += g.rows_step) {
         float x[VEC];
         load_input<T, VEC, MASK>(p, r * p.d + g.feature, x);
 #pragma unroll
-        for (int v = 0; v < VEC; ++v) x[v] = output(v, x[v]);
+        for (int v = 0; v < VEC; ++v) x[v] = output(far, feature, v, x[v]);
         Elem<T>::template store<VEC>(out + r * p.d + g.feature, x);
       }
     }
@@ -887,7 +887,7 @@ __device__ __forceinline__ bool finish_deferred(const Params& p, int64_t idx, in
   const int rstep = wave_rows ? kWave / g.lpr : g.rows_step;
   const int row0 = wave_rows ? (t / kWave) * RPT * rstep + (t % kWave) / g.lpr : g.row_lane;
   const int wave_row0 = wave_rows ? __builtin_amdgcn_readfirstlane((t / kWave) * RPT * rstep) : 0;
-  const int voff = g.active ? (row0 * p.d + g.feature) * (int)sizeof(T) : kOutOfRange;
+  int voff = g.active ? (row0 * p.d + g.feature) * (int)sizeof(T) : kOutOfRange;
   const int step = rstep * p.d * (int)sizeof(T);
   const int64_t elems = (int64_t)it.rows * p.d;
   const Rsrc in = make_rsrc(static_cast<const T*>(p.values) + it.start * p.d, elems * (int64_t)sizeof(T));
@@ -911,14 +911,17 @@ __device__ __forceinline__ bool finish_deferred(const Params& p, int64_t idx, in
       Reg::set(data[i], x);
     }
   }
-  column_constants();
+  const bool far = is_far();
   const Rsrc out = make_rsrc(static_cast<T*>(p.out) + it.start * p.d, elems * (int64_t)sizeof(T));
+  asm volatile("" : "+v"(voff));    // (the rows' offsets are computed again, not held)
 #pragma unroll
   for (int i = 0; i < RPT; ++i) {
     if (i != 0 && wave_row0 + i * rstep >= it.rows) continue;
+    int f = feature;
+    asm volatile("" : "+v"(f));
     float y[VEC];
 #pragma unroll
-    for (int v = 0; v < VEC; ++v) y[v] = output(v, Reg::get(data[i], v));
+    for (int v = 0; v < VEC; ++v) y[v] = output(far, f, v, Reg::get(data[i], v));
     uint32_t w[In::kCount];
     In::set(w, y);
     buffer_store<In::kBytes>(out, voff + i * step, 0, w);
