@@ -563,12 +563,14 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
       // row before: bf16 D=16, 1,000,003 rows, scale and mask, 107 -> 58 us a
       // call), and none of the next group's, which would take registers the
       // rows need (bf16 D=46, 500,000 rows, masked: 21 registers spilled, 118
-      // -> 102 us).
+      // -> 102 us). f32 at the base priority again (D=128, 262,144 rows, masked
+      // 135.2 -> 131.7 us); where one group holds every row, a row's mask and
+      // values issue together (f32 D=25 masked 88.7 -> 86.2 us with both).
       constexpr int kRawMost = VEC == 1 ? RPT : In::kCount > 2 ? 32 / In::kCount : 16;
       constexpr int kRawRows = kRawMost < RPT ? kRawMost : RPT;
-      __builtin_amdgcn_s_setprio(3);
-      if constexpr (MASK) {
-        const Rsrc mk = make_rsrc(p.mask + start * d, chunk_elems * 4);
+      if (!kAccurate) __builtin_amdgcn_s_setprio(3);
+      const Rsrc mk = make_rsrc(MASK ? p.mask + start * d : nullptr, MASK ? chunk_elems * 4 : 0);
+      if constexpr (MASK && kRawRows < RPT) {
 #pragma unroll
         for (int i = 0; i < RPT; ++i) buffer_load<VEC * 4>(mk, voff_m + i * step_mask, 0, data[i]);
       }
@@ -576,8 +578,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
       for (int i0 = 0; i0 < RPT; i0 += kRawRows) {
         uint32_t raw[kRawRows][In::kCount];
 #pragma unroll
-        for (int i = 0; i < kRawRows; ++i) buffer_load<In::kBytes>(in, voff + (i0 + i) * step_in, 0, raw[i]);
-        __builtin_amdgcn_s_setprio(0);
+        for (int i = 0; i < kRawRows; ++i) {
+          if constexpr (MASK && kRawRows == RPT) buffer_load<VEC * 4>(mk, voff_m + i * step_mask, 0, data[i]);
+          buffer_load<In::kBytes>(in, voff + (i0 + i) * step_in, 0, raw[i]);
+        }
+        if (!kAccurate) __builtin_amdgcn_s_setprio(0);
 #pragma unroll
         for (int i = 0; i < kRawRows; ++i) {
 #pragma clang fp contract(off)
