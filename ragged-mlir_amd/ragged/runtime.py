@@ -514,7 +514,9 @@ class CompiledProgram:
         torch = _torch_module
         if torch is None:
             return None
-        short = schedule is None and self._short_segments(max_len)
+        # (-1: known to have no such schedule; a method call less.)
+        short = (schedule is None and max_len is not None and self._short_limit != -1
+                 and self._short_segments(max_len))
         if schedule is None and not short and self._schedule == "classified" and self.spec.op != "softmax":
             return None        # the part size of its split segments: _run
         facts = self._tensor_facts(torch, values, offsets, out, mask)
@@ -531,7 +533,7 @@ class CompiledProgram:
             if short:
                 schedule = "short"
                 selection = {**selection, "short_segments": True}
-            elif self._holds(n, max_len):
+            elif self._held != -1 and self._holds(n, max_len):
                 schedule = "held"
         elif schedule != "tiles":
             return None
@@ -712,7 +714,7 @@ class CompiledProgram:
                     chosen, selection = self._reduce_route(values.shape[0], offsets.shape[0] - 1, max_len)
                 except (AttributeError, IndexError, TypeError):
                     chosen, selection = "classified", {"max_len": max_len, "tiles": True}     # validation reports it
-                if selection.get("tiles"):
+                if "tiles" in selection:
                     return self._run(values, offsets, out, stream, mode, debug_buffers=debug_buffers, mask=mask,
                                      selected="classified", selection=selection, schedule="tiles")
             elif self._short_segments(max_len):
