@@ -199,16 +199,32 @@ __device__ __forceinline__ void normalize_flat(const Params& p, int g, int t, in
 }
 
 // In FLAT mode component c holds feature c % D (D a power of two dividing
-// VEC): fold components D.. into 0..D-1, each target in increasing c. The
-// target is selected among the constant indices t < c, so no register
-// array is indexed by a run-time value (which would place it in scratch).
+// VEC): fold components D.. into 0..D-1, each target in increasing c (sums: by
+// halves, in f64). The target is selected among constant indices, so no
+// register array is indexed by a run-time value (which would place it in
+// scratch).
 template <int OP, int VEC>
 __device__ __forceinline__ void merge_components(State<OP> (&st)[VEC], int d) {
+  if constexpr (OP == OP_SUM) {
+    double x[VEC];
 #pragma unroll
-  for (int c = 1; c < VEC; ++c) {
+    for (int c = 0; c < VEC; ++c) x[c] = sum_f64(st[c]);
 #pragma unroll
-    for (int t = 0; t < c; ++t) {
-      if (c >= d && (c & (d - 1)) == t) merge_exact<OP>(st[t], st[c]);
+    for (int off = VEC / 2; off >= 1; off /= 2) {
+      if (off >= d) {
+#pragma unroll
+        for (int c = 0; c < off; ++c) x[c] += x[c + off];
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < VEC; ++c) st[c] = sum_state(x[c]);
+  } else {
+#pragma unroll
+    for (int c = 1; c < VEC; ++c) {
+#pragma unroll
+      for (int t = 0; t < c; ++t) {
+        if (c >= d && (c & (d - 1)) == t) st[t].merge(st[c]);
+      }
     }
   }
 }
@@ -231,11 +247,13 @@ __device__ __forceinline__ void spread_components(float (&x)[VEC], int d) {
 // lanes agree modulo `lpr`. Every thread ends with the total for its own
 // feature lane. `lds` holds kBlock * VEC * 2 floats.
 
+// Only the first `count` components matter (flat mapping: D of them).
+
 template <int OP, int VEC>
-__device__ __forceinline__ void block_reduce(State<OP> (&st)[VEC], int lpr, int feat_lane, float* lds) {
+__device__ __forceinline__ void block_reduce(State<OP> (&st)[VEC], int lpr, int feat_lane, float* lds, int count = VEC) {
   constexpr int S = Slots<OP>::kCount;
   const int t = threadIdx.x, lane = t & (kWave - 1), w = t / kWave;
-  if (lpr < kWave) wave_reduce_stride<OP, VEC>(st, lpr);
+  if (lpr < kWave) wave_reduce_stride<OP, VEC>(st, lpr, count);
   const int rep = lpr < kWave ? lpr : kWave;
   if (lane < rep) {
 #pragma unroll
@@ -243,24 +261,30 @@ __device__ __forceinline__ void block_reduce(State<OP> (&st)[VEC], int lpr, int 
   }
   __syncthreads();
   State<OP> acc[VEC];
-  if (t < lpr) {
-    if (lpr <= kWave) {
+  // Waves `first`, first + step, ... of lane l, in order.
+  auto fold_waves = [&](int first, int step, int l) {
 #pragma unroll
-      for (int v = 0; v < VEC; ++v) acc[v] = st_read<OP>(lds + (t * VEC + v) * S, 1);
-      for (int ww = 1; ww < kWavesPerBlock; ++ww) {
+    for (int v = 0; v < VEC; ++v) acc[v] = st_read<OP>(lds + ((first * kWave + l) * VEC + v) * S, 1);
+    if constexpr (OP == OP_SUM) {
+      double x[VEC];
 #pragma unroll
-        for (int v = 0; v < VEC; ++v) merge_exact<OP>(acc[v], st_read<OP>(lds + ((ww * kWave + t) * VEC + v) * S, 1));
+      for (int v = 0; v < VEC; ++v) x[v] = acc[v].s;
+      for (int ww = first + step; ww < kWavesPerBlock; ww += step) {
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) x[v] += lds[(ww * kWave + l) * VEC + v];
       }
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) acc[v].s = (float)x[v];
     } else {
-      const int wpr = lpr / kWave;              // waves per row
-      const int w0 = t / kWave, l0 = t & (kWave - 1);
+      for (int ww = first + step; ww < kWavesPerBlock; ww += step) {
 #pragma unroll
-      for (int v = 0; v < VEC; ++v) acc[v] = st_read<OP>(lds + ((w0 * kWave + l0) * VEC + v) * S, 1);
-      for (int ww = w0 + wpr; ww < kWavesPerBlock; ww += wpr) {
-#pragma unroll
-        for (int v = 0; v < VEC; ++v) merge_exact<OP>(acc[v], st_read<OP>(lds + ((ww * kWave + l0) * VEC + v) * S, 1));
+        for (int v = 0; v < VEC; ++v) acc[v].merge(st_read<OP>(lds + ((ww * kWave + l) * VEC + v) * S, 1));
       }
     }
+  };
+  if (t < lpr) {
+    if (lpr <= kWave) fold_waves(0, 1, t);
+    else fold_waves(t / kWave, lpr / kWave, t & (kWave - 1));      // lpr / 64 waves per row
   }
   __syncthreads();
   if (t < lpr) {
@@ -407,8 +431,9 @@ __device__ __forceinline__ void process_segment(const Params& p, int64_t s, int6
     const int64_t lo = start * p.d, hi = end * p.d;
     fold_flat<OP, T, VEC, MASK>(p, G, t, lo, hi, st);
     merge_components<OP, VEC>(st, p.d);
-    if constexpr (BLOCK) block_reduce<OP, VEC>(st, 1, 0, lds);
-    else wave_reduce_stride<OP, VEC>(st, 1);
+    const int count = OP == OP_SUM ? p.d : VEC;
+    if constexpr (BLOCK) block_reduce<OP, VEC>(st, 1, 0, lds, count);
+    else wave_reduce_stride<OP, VEC>(st, 1, count);
     if constexpr (OP == OP_SOFTMAX) {
       float m[VEC], inv[VEC];
       softmax_factors<VEC>(st, m, inv);

@@ -173,9 +173,9 @@ __device__ __forceinline__ void fold_tiles(const Params& p, int64_t tile0, int l
     if (parts_of(k) > kFoldWave * in_wave) continue;
     State<OP> acc;
     shared(acc, k, (t & (kWave - 1)) / lanes, in_wave);
-    xor_butterfly_range(lanes, kWave, [&](auto mask) {
-      merge_exact<OP>(acc, shfl_xor_exact<decltype(mask)::value, OP>(acc));
-    });
+    State<OP> one[1] = {acc};
+    merge_lanes<OP, 1>(one, [&](auto&& step) { xor_butterfly_range(lanes, kWave, step); });
+    acc = one[0];
     if ((t & (kWave - 1)) < lanes && f < d) finish(acc, k);
   }
   for (int k = 0; k < many; ++k) {
@@ -274,10 +274,7 @@ __global__ __launch_bounds__(kTileThreads) void k_tiles(Params p) {
 
     // The states of `lanes` row lanes into one.
     auto reduce = [&](int lanes) {
-      xor_butterfly_range(lpr, lpr * lanes, [&](auto mask) {
-#pragma unroll
-        for (int v = 0; v < VEC; ++v) merge_exact<OP>(st[v], shfl_xor_exact<decltype(mask)::value, OP>(st[v]));
-      });
+      if (lanes > 1) merge_lanes<OP, VEC>(st, [&](auto&& step) { xor_butterfly_range(lpr, lpr * lanes, step); });
     };
     auto put_partial = [&](int which) {
       if (!p.partials) return;      // a single tile has none (valid offsets)

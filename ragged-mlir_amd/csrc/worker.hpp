@@ -365,7 +365,7 @@ __device__ __forceinline__ void split_part(const Params& p, int64_t item, int ti
   if constexpr (FLAT) {
     fold_flat<OP, T, VEC, MASK>(p, kBlock, t, start * p.d, end * p.d, st);
     merge_components<OP, VEC>(st, p.d);
-    block_reduce<OP, VEC>(st, 1, 0, lds);
+    block_reduce<OP, VEC>(st, 1, 0, lds, OP == OP_SUM ? p.d : VEC);
     if (t == 0) {
 #pragma unroll
       for (int f = 0; f < VEC; ++f) {
