@@ -522,24 +522,40 @@ __device__ __forceinline__ double xor_lane_f64(double v) {
 }
 
 // Combine lanes over the masks `butterfly` applies (xor_butterfly and its
-// like), the first `count` of the V states. Sums go through f64, which keeps
-// the rounding of every addition for one v_add_f64 a step; two-sums in f32 (ten
-// operations and a test for infinities) took block-per-segment sums from 13.5 to
-// 25.8 us (f32 D=1, 10,000 segments of 64 rows), 17.6 to 46.2 (bf16 D=1).
-template <int OP, int V, class Butterfly>
+// like), the first `count` of the V states. F64: sums go through f64, which
+// keeps the rounding of every addition for one v_add_f64 a step; two-sums in f32
+// (ten operations and a test for infinities) took block-per-segment sums from
+// 13.5 to 25.8 us (f32 D=1, 10,000 segments of 64 rows). bf16 results, whose
+// rounding is 2^16 times coarser, merge in f32 (bf16 D=4, 10,000 segments 27.0
+// us in f64, 17.9 so).
+template <int OP, int V, bool F64, class Butterfly>
 __device__ __forceinline__ void merge_lanes(State<OP> (&st)[V], Butterfly&& butterfly, int count = V) {
   if constexpr (OP == OP_SUM) {
-    double x[V];
+    using X = typename std::conditional<F64, double, float>::type;
+    X x[V];
 #pragma unroll
-    for (int v = 0; v < V; ++v) x[v] = sum_f64(st[v]);
+    for (int v = 0; v < V; ++v) {
+      if constexpr (F64) x[v] = sum_f64(st[v]);
+      else x[v] = st[v].s - st[v].c;
+    }
     butterfly([&](auto mask) {
 #pragma unroll
       for (int v = 0; v < V; ++v) {
-        if (v < count) x[v] += xor_lane_f64<decltype(mask)::value>(x[v]);
+        if (v < count) {
+          if constexpr (F64) x[v] += xor_lane_f64<decltype(mask)::value>(x[v]);
+          else x[v] += xor_lane<decltype(mask)::value>(x[v]);
+        }
       }
     });
 #pragma unroll
-    for (int v = 0; v < V; ++v) st[v] = sum_state(x[v]);
+    for (int v = 0; v < V; ++v) {
+      if constexpr (F64) {
+        st[v] = sum_state(x[v]);
+      } else {
+        st[v].s = x[v];
+        st[v].c = 0.f;
+      }
+    }
   } else {
     butterfly([&](auto mask) {
 #pragma unroll
@@ -550,9 +566,9 @@ __device__ __forceinline__ void merge_lanes(State<OP> (&st)[V], Butterfly&& butt
 
 // Combine lanes whose lane index agrees modulo `stride` (a power of two < 64):
 // afterwards every lane holds the combination over its residue class.
-template <int OP, int V>
+template <int OP, int V, bool F64 = true>
 __device__ __forceinline__ void wave_reduce_stride(State<OP> (&st)[V], int stride, int count = V) {
-  merge_lanes<OP, V>(st, [&](auto&& step) { xor_butterfly(stride, step); }, count);
+  merge_lanes<OP, V, F64>(st, [&](auto&& step) { xor_butterfly(stride, step); }, count);
   if constexpr (OP == OP_SUM) {
 #pragma unroll
     for (int v = 0; v < V; ++v) st[v].c = 0.f;

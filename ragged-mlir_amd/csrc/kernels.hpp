@@ -249,11 +249,11 @@ __device__ __forceinline__ void spread_components(float (&x)[VEC], int d) {
 
 // Only the first `count` components matter (flat mapping: D of them).
 
-template <int OP, int VEC>
+template <int OP, int VEC, bool F64 = true>
 __device__ __forceinline__ void block_reduce(State<OP> (&st)[VEC], int lpr, int feat_lane, float* lds, int count = VEC) {
   constexpr int S = Slots<OP>::kCount;
   const int t = threadIdx.x, lane = t & (kWave - 1), w = t / kWave;
-  if (lpr < kWave) wave_reduce_stride<OP, VEC>(st, lpr, count);
+  if (lpr < kWave) wave_reduce_stride<OP, VEC, F64>(st, lpr, count);
   const int rep = lpr < kWave ? lpr : kWave;
   if (lane < rep) {
 #pragma unroll
@@ -266,7 +266,7 @@ __device__ __forceinline__ void block_reduce(State<OP> (&st)[VEC], int lpr, int 
 #pragma unroll
     for (int v = 0; v < VEC; ++v) acc[v] = st_read<OP>(lds + ((first * kWave + l) * VEC + v) * S, 1);
     if constexpr (OP == OP_SUM) {
-      double x[VEC];
+      typename std::conditional<F64, double, float>::type x[VEC];
 #pragma unroll
       for (int v = 0; v < VEC; ++v) x[v] = acc[v].s;
       for (int ww = first + step; ww < kWavesPerBlock; ww += step) {
@@ -418,6 +418,7 @@ template <int OP, class T, int VEC, bool FLAT, bool MASK, bool BLOCK, bool HELD 
 __device__ __forceinline__ void process_segment(const Params& p, int64_t s, int64_t start, int64_t end,
                                                 int tile, float* lds) {
   constexpr int G = BLOCK ? kBlock : kWave;
+  constexpr bool kF64 = std::is_same<T, float>::value;      // sums of f32 results (merge_lanes)
   const int t = BLOCK ? threadIdx.x : (threadIdx.x & (kWave - 1));
   if constexpr (OP == OP_SOFTMAX && BLOCK && HELD && !MASK) {
     if (held_softmax<T, VEC, FLAT>(p, start, end, tile, lds)) {
@@ -432,8 +433,8 @@ __device__ __forceinline__ void process_segment(const Params& p, int64_t s, int6
     fold_flat<OP, T, VEC, MASK>(p, G, t, lo, hi, st);
     merge_components<OP, VEC>(st, p.d);
     const int count = OP == OP_SUM ? p.d : VEC;
-    if constexpr (BLOCK) block_reduce<OP, VEC>(st, 1, 0, lds, count);
-    else wave_reduce_stride<OP, VEC>(st, 1, count);
+    if constexpr (BLOCK) block_reduce<OP, VEC, kF64>(st, 1, 0, lds, count);
+    else wave_reduce_stride<OP, VEC, kF64>(st, 1, count);
     if constexpr (OP == OP_SOFTMAX) {
       float m[VEC], inv[VEC];
       softmax_factors<VEC>(st, m, inv);
@@ -453,8 +454,8 @@ __device__ __forceinline__ void process_segment(const Params& p, int64_t s, int6
   } else {
     const RowGeo g = row_geo<VEC>(p.d, G, t, tile);
     fold_rows<OP, T, VEC, MASK>(p, g, start, end, st);
-    if constexpr (BLOCK) block_reduce<OP, VEC>(st, g.lpr, g.feat_lane, lds);
-    else if (g.lpr < kWave) wave_reduce_stride<OP, VEC>(st, g.lpr);
+    if constexpr (BLOCK) block_reduce<OP, VEC, kF64>(st, g.lpr, g.feat_lane, lds);
+    else if (g.lpr < kWave) wave_reduce_stride<OP, VEC, kF64>(st, g.lpr);
     if constexpr (OP == OP_SOFTMAX) {
       float m[VEC], inv[VEC];
       softmax_factors<VEC>(st, m, inv);

@@ -174,7 +174,7 @@ __device__ __forceinline__ void fold_tiles(const Params& p, int64_t tile0, int l
     State<OP> acc;
     shared(acc, k, (t & (kWave - 1)) / lanes, in_wave);
     State<OP> one[1] = {acc};
-    merge_lanes<OP, 1>(one, [&](auto&& step) { xor_butterfly_range(lanes, kWave, step); });
+    merge_lanes<OP, 1, true>(one, [&](auto&& step) { xor_butterfly_range(lanes, kWave, step); });
     acc = one[0];
     if ((t & (kWave - 1)) < lanes && f < d) finish(acc, k);
   }
@@ -274,7 +274,7 @@ __global__ __launch_bounds__(kTileThreads) void k_tiles(Params p) {
 
     // The states of `lanes` row lanes into one.
     auto reduce = [&](int lanes) {
-      if (lanes > 1) merge_lanes<OP, VEC>(st, [&](auto&& step) { xor_butterfly_range(lpr, lpr * lanes, step); });
+      if (lanes > 1) merge_lanes<OP, VEC, true>(st, [&](auto&& step) { xor_butterfly_range(lpr, lpr * lanes, step); });
     };
     auto put_partial = [&](int which) {
       if (!p.partials) return;      // a single tile has none (valid offsets)

@@ -344,7 +344,8 @@ __device__ __forceinline__ void group_segment(const Params& p, int64_t s, int64_
         for (int v = 0; v < VEC; ++v) st[v].fold(x[v]);
       });
       float y[VEC];
-      result_of<OP, VEC>(st, y);
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) y[v] = exact_value<OP>(st[v]);
       Elem<T>::template store<VEC>(static_cast<T*>(p.out) + s * d + f0, y);
     }
   }
