@@ -527,7 +527,7 @@ __device__ __forceinline__ double xor_lane_f64(double v) {
 // (ten operations and a test for infinities) took block-per-segment sums from
 // 13.5 to 25.8 us (f32 D=1, 10,000 segments of 64 rows). bf16 results, whose
 // rounding is 2^16 times coarser, merge in f32 (bf16 D=4, 10,000 segments 27.0
-// us in f64, 17.9 so).
+// us in f64, 21.1 so).
 template <int OP, int V, bool F64, class Butterfly>
 __device__ __forceinline__ void merge_lanes(State<OP> (&st)[V], Butterfly&& butterfly, int count = V) {
   if constexpr (OP == OP_SUM) {

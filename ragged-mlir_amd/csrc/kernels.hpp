@@ -247,8 +247,8 @@ __device__ __forceinline__ void spread_components(float (&x)[VEC], int d) {
 // lanes agree modulo `lpr`. Every thread ends with the total for its own
 // feature lane. `lds` holds kBlock * VEC * 2 floats.
 
-// Only the first `count` components matter (flat mapping: D of them).
-
+// Only the first `count` components matter (flat mapping: D of them). F64: as in
+// merge_lanes.
 template <int OP, int VEC, bool F64 = true>
 __device__ __forceinline__ void block_reduce(State<OP> (&st)[VEC], int lpr, int feat_lane, float* lds, int count = VEC) {
   constexpr int S = Slots<OP>::kCount;
